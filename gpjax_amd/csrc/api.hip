@@ -119,7 +119,6 @@ int decode_prec(int prec, Arith3* ar) {
 
 struct Layout {
   int64_t np = 0;
-  int64_t htop = 0;
   size_t ts = 0;
   size_t off_L = 0, off_X = 0, off_T = 0, off_leafinv = 0, off_leafld = 0, off_leafinfo = 0;
   // r, alpha, u and v each lead a block of nvec vectors (np apart): with the
@@ -143,7 +142,6 @@ Layout make_layout(int64_t n, int64_t d, int prec, int spk = -1) {
   L.np = round_up(n, NB);
   L.ts = prec == GPK_PREC_FP64 ? sizeof(double) : sizeof(float);
   const int64_t np = L.np;
-  L.htop = np > NB ? split_point(np) : 0;
   const int64_t nleaf = np / NB;
   const int64_t ntile = nleaf * (nleaf + 1) / 2;
   // partial sums of the triangular matvecs (1,024-row chunks) and of the
@@ -152,7 +150,7 @@ Layout make_layout(int64_t n, int64_t d, int prec, int spk = -1) {
   size_t o = 0;
   L.off_L = o; o += al((size_t)np * np * L.ts);
   L.off_X = o; o += al((size_t)np * np * L.ts);
-  L.off_T = o; o += al((size_t)(np - L.htop) * (L.htop > 0 ? L.htop : 1) * L.ts);
+  L.off_T = o; o += al((size_t)factor_scratch_elems(np) * L.ts);
   L.off_leafinv = o; o += al((size_t)np * NB * sizeof(double));
   L.off_leafld = o; o += al((size_t)nleaf * sizeof(double));
   L.off_leafinfo = o; o += al((size_t)nleaf * sizeof(int));

@@ -23,6 +23,12 @@ namespace gpk {
 
 inline int64_t split_point(int64_t n) { return (n / NB / 2) * NB; }
 
+// 128-row blocks x members up to which a triangular solve's leaf runs in strips
+// (wide batches take the 128 x 128 tiles: 4,096 small GPs 62.3 -> 61.1 ms).
+constexpr int64_t TRSM_STRIP_TILES = 512;
+static_assert(TRSM_STRIP_TILES >= SMALL_TILES, "an in-place product on small tiles would race");
+constexpr unsigned TRI_NODEWISE = 64;  // members from which the inverse goes node by node
+
 // Panel width of the look-ahead Cholesky (Factor::potrf_lookahead) for a single
 // np x np problem, np >= 2,048: np/32 with float32 storage, np/64 in float64,
 // rounded down to a multiple of NB, at least NB.  Wider panels put more of the
@@ -46,6 +52,26 @@ inline int64_t lookahead_width(int64_t np, bool f32) {
   if (np < 2048) return 0;
   const int64_t b = (np / (f32 ? 32 : 64)) / NB * NB;
   return b < NB ? NB : b;
+}
+
+// Depth of the triangular inverse's recursion over n rows with leaves of `unit`.
+inline int tri_depth(int n, int unit) {
+  int d = 0;
+  while (n > unit) {
+    n -= tri_split(n, unit);  // the larger half
+    ++d;
+  }
+  return d;
+}
+// Largest T (rows, columns) of a level's nodes.
+inline void tri_extents(const TriLevel& lev, int& mm, int& mn) {
+  mm = mn = 0;
+  for (unsigned q = 0; q < lev.nodes; ++q) {
+    int o, n, h;
+    if (!tri_node(lev, q, o, n, h)) continue;
+    if (n - h > mm) mm = n - h;
+    if (h > mn) mn = h;
+  }
 }
 
 template <typename T>
@@ -97,6 +123,12 @@ struct Factor {
                                        fscale ? fscale + 1 : nullptr);
       }
       const double* inv = leafinv + (o / NB) * NB * NB;
+      if constexpr (std::is_same<TS, double>::value) {
+        if (m / NB * bt.count <= TRSM_STRIP_TILES)
+          return launch_trsm_strip(L + row0 * ld + o, ld, m, inv, s, bt);
+      }
+      // In place: a workgroup must own its rows' NB columns, so this launch must
+      // not take the FP64 products' smaller tiles (it has more tiles than they do).
       return launch_gemm<TS, double, TS>(AR_F64, false, false, L + row0 * ld + o, ld, inv, NB,
                                          L + row0 * ld + o, ld, m, NB, NB, 1.0, false, false,
                                          KR_FULL, s, nullptr, bt);
@@ -175,29 +207,79 @@ struct Factor {
     tri_unit = B;
     return GPK_OK;
   }
-  // X = L^-1 below the leaves, whose diagonal blocks the leaves already wrote.
+  // X = L^-1 below the leaves, whose diagonal blocks the leaves already wrote:
+  // level by level from the deepest, all nodes of a level (independent of each
+  // other) in one launch per product, or for a wide batch, whose single nodes
+  // fill the chip, node by node (a node's T and X are then still in cache when its
+  // second product and its parent read them: 4,096 small GPs 61.7 -> 60.2 ms).
+  // n = 2,000: 30 launches of one to 64 workgroups 1,217 us, eight launches 195 us.
   int trtri(int64_t o, int64_t n) {
-    if (n <= tri_unit) return GPK_OK;
-    const int64_t hu = n / tri_unit / 2;
-    const int64_t h = (hu > 0 ? hu : 1) * tri_unit;
-    GPK_TRY(trtri(o, h));
-    GPK_TRY(trtri(o + h, n - h));
+    const int depth = tri_depth((int)n, (int)tri_unit);
+    if (bt.count >= TRI_NODEWISE) return trtri_node(o, n, 0, 0);
+    for (int d = depth - 1; d >= 0; --d) GPK_TRY(trtri_level(o, n, d, 0, 1u << d));
+    return GPK_OK;
+  }
+  // Nodes first .. first + count - 1 of a level of the inverse over rows o .. o + n.
+  int trtri_level(int64_t o, int64_t n, int depth, unsigned first, unsigned count) {
+    TriLevel lev;
+    lev.nodes = 1u << depth;
+    lev.depth = depth;
+    lev.o = (int)o;
+    lev.n = (int)n;
+    lev.unit = (int)tri_unit;
+    lev.ld = (int)ld;
+    int mm, mn;
+    tri_extents(lev, mm, mn);
+    lev.tstride = depth == 0 ? 0 : mn;
+    lev.first = first;
+    lev.nodes = count;
     // T = L21 X11   ((n-h) x h; X11 lower, so k >= column tile)
-    GPK_TRY(launch_gemm<TS, TS, TS>(ar_trtri, false, true, L + (o + h) * ld + o, ld,
-                                    X + o * ld + o, ld, T, h, n - h, h, h, 1.0, false, false,
-                                    KR_GE_N, s, nullptr, bt, fscale ? fscale + 1 : nullptr));
+    lev.product = 1;
+    GPK_TRY(launch_tri_level<TS>(ar_trtri, lev, mm, mn, L, ld, X, ld, T, mn, s, bt,
+                                 fscale ? fscale + 1 : nullptr));
     // X21 = -X22 T  (X22 lower, so k <= row tile)
-    return launch_gemm<TS, TS, TS>(ar_trtri, false, true, X + (o + h) * ld + o + h, ld, T, h,
-                                   X + (o + h) * ld + o, ld, n - h, h, n - h, -1.0, false,
-                                   false, KR_LE_M, s, nullptr, bt,
-                                   fscale ? fscale + 2 : nullptr);
+    lev.product = 2;
+    return launch_tri_level<TS>(ar_trtri, lev, mm, mn, X, ld, T, mn, X, ld, s, bt,
+                                fscale ? fscale + 2 : nullptr);
+  }
+  int trtri_node(int64_t o, int64_t n, unsigned path, int d) {
+    TriLevel lev;
+    lev.depth = d;
+    lev.o = (int)o;
+    lev.n = (int)n;
+    lev.unit = (int)tri_unit;
+    int no, nn, h;
+    if (!tri_node(lev, path, no, nn, h)) return GPK_OK;
+    GPK_TRY(trtri_node(o, n, 2 * path, d + 1));
+    GPK_TRY(trtri_node(o, n, 2 * path + 1, d + 1));
+    return trtri_level(o, n, d, path, 1);
   }
 };
 
-// Elements of the trtri scratch T for an n x n factorisation.
+// Elements of the trtri scratch T for an n x n factorisation: the largest level's,
+// for either width of its leaves.
 inline int64_t factor_scratch_elems(int64_t n) {
-  const int64_t h = n > NB ? split_point(n) : 1;
-  return (n - h) * h;
+  int64_t best = 1;
+  for (const int64_t unit : {(int64_t)NB, lookahead_width(n, false), lookahead_width(n, true)}) {
+    if (unit <= 0) continue;
+    for (int depth = tri_depth((int)n, (int)unit) - 1; depth >= 0; --depth) {
+      TriLevel lev;
+      lev.nodes = 1u << depth;
+      lev.depth = depth;
+      lev.n = (int)n;
+      lev.unit = (int)unit;
+      int mm, mn;
+      tri_extents(lev, mm, mn);
+      const int64_t stride = depth == 0 ? 0 : mn;
+      for (unsigned q = 0; q < lev.nodes; ++q) {
+        int o, nn, h;
+        if (!tri_node(lev, q, o, nn, h)) continue;
+        const int64_t end = o * stride + (int64_t)(nn - h) * h;
+        if (end > best) best = end;
+      }
+    }
+  }
+  return best;
 }
 
 }  // namespace gpk

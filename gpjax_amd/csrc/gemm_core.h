@@ -449,14 +449,19 @@ __device__ __forceinline__ int acc_row(int lane, int r) {
   return AR == AR_F64 ? (lane >> 4) + 4 * r : 4 * (lane >> 4) + r;
 }
 
+// The tile decodes below work in 32 bits (a launch has fewer than 2^31 tiles): a
+// 64-bit quotient is a call-sized sequence in every workgroup's prologue.
+//
 // Tile decode for lower-triangular tile sets: t -> (mt, nt), mt >= nt, with
 // tiles of small mt first.
-__device__ __forceinline__ void lower_tile(int64_t t, int64_t& mt, int64_t& nt) {
-  int64_t a = (int64_t)((sqrt(8.0 * (double)t + 1.0) - 1.0) * 0.5);
-  while (a * (a + 1) / 2 > t) --a;
-  while ((a + 1) * (a + 2) / 2 <= t) ++a;
+__device__ __forceinline__ void lower_tile(int64_t t64, int64_t& mt, int64_t& nt) {
+  const int t = (int)t64;
+  int a = (int)((sqrt(8.0 * (double)t + 1.0) - 1.0) * 0.5);
+  auto tri = [](int v) { return (int)((unsigned)v * (unsigned)(v + 1) / 2u); };
+  while (tri(a) > t) --a;
+  while (tri(a + 1) <= t) ++a;
   mt = a;
-  nt = t - a * (a + 1) / 2;
+  nt = t - tri(a);
 }
 
 // Tile decode for a lower-triangular tile set of T x T tiles in bands: rows
@@ -465,18 +470,19 @@ __device__ __forceinline__ void lower_tile(int64_t t, int64_t& mt, int64_t& nt) 
 // time (row-major within each 16-column block, the diagonal block last).  About
 // 256 consecutive tiles, the ones resident at a time, then share 16 row and 16
 // column operand panels instead of one row panel and 256 column panels.
-__device__ __forceinline__ void lower_tile_banded(int64_t t, int64_t T, int64_t& mt,
+__device__ __forceinline__ void lower_tile_banded(int64_t t64, int64_t T64, int64_t& mt,
                                                   int64_t& nt) {
-  constexpr int64_t H = 16;
-  auto cum = [](int64_t S) { return 128 * S * (S - 1) + 136 * S; };  // tiles of full bands < S
-  int64_t S = (int64_t)((-8.0 + sqrt(64.0 + 512.0 * (double)t)) / 256.0);
+  constexpr int H = 16;
+  const int t = (int)t64, T = (int)T64;
+  auto cum = [](int S) { return 128 * S * (S - 1) + 136 * S; };  // tiles of full bands < S
+  int S = (int)((-8.0 + sqrt(64.0 + 512.0 * (double)t)) / 256.0);
   while (S > 0 && cum(S) > t) --S;
   while (cum(S + 1) <= t && H * (S + 1) < T) ++S;
-  const int64_t R0 = H * S;
-  const int64_t h = (T - R0 < H) ? T - R0 : H;
-  const int64_t u = t - cum(S);
+  const int R0 = H * S;
+  const unsigned h = (T - R0 < H) ? T - R0 : H;
+  const unsigned u = t - cum(S);
   if (u < S * H * h) {
-    const int64_t cb = u / (H * h), v = u % (H * h);
+    const unsigned cb = u / (H * h), v = u % (H * h);
     mt = R0 + v / H;
     nt = H * cb + v % H;
   } else {
@@ -490,15 +496,16 @@ __device__ __forceinline__ void lower_tile_banded(int64_t t, int64_t T, int64_t&
 // The same for a full Mt x Nt tile grid: b (row-major launch order) -> bands of
 // 16 tile rows from the top, 16-column blocks within a band, row-major within
 // a block (ragged last band and block included).
-__device__ __forceinline__ void grid_tile_banded(int64_t b, int64_t Mt, int64_t Nt, int64_t& mt,
-                                                 int64_t& nt) {
-  constexpr int64_t H = 16;
-  const int64_t S = b / (H * Nt);
-  const int64_t u = b - S * H * Nt;
-  const int64_t h = (Mt - S * H < H) ? Mt - S * H : H;
-  const int64_t cb = u / (h * H);
-  const int64_t v = u - cb * h * H;
-  const int64_t w = (Nt - H * cb < H) ? Nt - H * cb : H;
+__device__ __forceinline__ void grid_tile_banded(int64_t b64, int64_t Mt64, int64_t Nt64,
+                                                 int64_t& mt, int64_t& nt) {
+  constexpr unsigned H = 16;
+  const unsigned b = (unsigned)b64, Mt = (unsigned)Mt64, Nt = (unsigned)Nt64;
+  const unsigned S = b / (H * Nt);
+  const unsigned u = b - S * H * Nt;
+  const unsigned h = (Mt - S * H < H) ? Mt - S * H : H;
+  const unsigned cb = u / (h * H);
+  const unsigned v = u - cb * h * H;
+  const unsigned w = (Nt - H * cb < H) ? Nt - H * cb : H;
   mt = S * H + v / w;
   nt = H * cb + v % w;
 }

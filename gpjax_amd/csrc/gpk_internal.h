@@ -240,6 +240,17 @@ enum KRange { KR_FULL = 0, KR_GE_N = 1, KR_LE_M = 2, KR_GE_M = 3 };
 // into fp16 hi + lo planes, products hi*hi + hi*lo + lo*hi.
 enum Arith { AR_F64 = 0, AR_BF16X3 = 3, AR_FP16X3 = 4, AR_BF16X6 = 6 };
 
+// Tile rule of the FP64 products (double operands, no diagonal side buffer), by the
+// number of 128-tiles of the launch: up to SMALL_TILES run on 64 x 64 tiles, up to
+// TINY_TILES on 32 x 32.  The line lies where 128-tiles fill the chip's two
+// workgroups per CU; MLL + gradient at n = 5,000: 6.57 ms with 160, 6.45 with 384,
+// 6.19 with 512, 6.27 with 1,024 (10.9 without), n = 16,384: 86.5 / 86.8 / 86.7 /
+// 87.3 (100.9).  TINY_TILES 8, 24 and 64 are within 1 %.  In a batch the other
+// pieces' launches fill the chip, so there only launches of few tiles take the small
+// ones (512 GPs of up to 600 rows: 3.17 ms with 512, 2.96 with 96).
+constexpr int64_t SMALL_TILES = 512, SMALL_TILES_BATCH = 96;
+constexpr int64_t TINY_TILES = 24;
+
 // C[M x N] = alpha * sum_k A(m, k) B(n, k) (+ C if beta_one), M, N, K multiples
 // of NB.  A(m, k) is A[m*lda + k] (a_km = false) or A[k*lda + m] (a_km = true);
 // B(n, k) is B[n*ldb + k] (b_kn = false) or B[k*ldb + n] (b_kn = true).
@@ -251,6 +262,52 @@ int launch_gemm(int arith, bool a_km, bool b_kn, const TA* A, int64_t lda, const
                 bool beta_one, bool lower_tiles, int krange, hipStream_t s,
                 double* cdiag = nullptr, const Batch& bt = Batch(),
                 const float* fscale = nullptr);
+
+// One level of the recursive triangular inverse as one launch: the 2^depth nodes of
+// that depth of the recursion over rows o .. o + n (splits as tri_split), a node
+// per z index.  Every node wider than `unit` computes T = L21 X11 (product 1) or
+// X21 = -X22 T (product 2); its T sits at T + (node's o - o) * tstride.
+struct TriLevel {
+  unsigned nodes = 0;  // nodes of this launch; 0: not a level of the inverse
+  unsigned first = 0;  // the first of them
+  int depth = 0;
+  int product = 0;
+  int o = 0, n = 0, unit = NB;  // 32 bits: a kernel argument of every tile GEMM
+  int ld = 0, tstride = 0;
+};
+__host__ __device__ inline int tri_split(int n, int unit) {
+  const int hu = n / unit / 2;
+  return (hu > 0 ? hu : 1) * unit;
+}
+// Node `node` of the level: rows o .. o + n, split at h; false if it is a leaf (or
+// below one).
+__host__ __device__ inline bool tri_node(const TriLevel& t, unsigned node, int& o, int& n,
+                                         int& h) {
+  o = t.o;
+  n = t.n;
+  for (int d = t.depth - 1; d >= 0; --d) {
+    if (n <= t.unit) return false;
+    h = tri_split(n, t.unit);
+    if ((node >> d) & 1) {
+      o += h;
+      n -= h;
+    } else {
+      n = h;
+    }
+  }
+  if (n <= t.unit) return false;
+  h = tri_split(n, t.unit);
+  return true;
+}
+// max_m x max_n: the largest node's T.  A, B, C as the product names them.
+template <typename TS>
+int launch_tri_level(int arith, const TriLevel& lev, int64_t max_m, int64_t max_n, const TS* A,
+                     int64_t lda, const TS* B, int64_t ldb, TS* C, int64_t ldc, hipStream_t s,
+                     const Batch& bt, const float* fscale);
+
+// Y = B L11^-T in place: m rows x NB columns (float64), inv = L11^-1 (NB x NB).
+int launch_trsm_strip(double* B, int64_t ld, int64_t m, const double* inv, hipStream_t s,
+                      const Batch& bt = Batch());
 
 // Fused LAUUM + adjoint: for every lower NB-tile of Sinv = X^T X (X = L^-1,
 // lower, Np x Np), reduce 1/2 tr(W dSigma/dtheta) contributions with
