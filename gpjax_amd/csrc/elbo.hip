@@ -40,7 +40,15 @@ constexpr int EDMAX = 32;   // largest input dimension on the ELBO path
 // chip (see S below): 231 -> 228 ms (FP64) and 83.3 -> 82.8 ms (mixed) at
 // N = 1e6, M = 2,048, for 2 GB more workspace.
 constexpr int64_t BW_CHUNK = 131072;
-constexpr int64_t EW = 1024;         // points per block of the gradient data pass
+// Points per block of the gradient data pass: the widest of 1,024 .. 128 whose grid
+// (row tiles x point blocks) has at least 1,024 workgroups.  Each block leaves
+// partial sums, so wide ones are the better as long as the chip is full
+// (n = 50,021, m = 500: 1,024 points 281 us on 196 workgroups, 128 points 136 us).
+inline int64_t wgrad_points(int64_t n, int64_t mt) {
+  int64_t ew = 1024;
+  while (ew > 128 && mt * ((n + ew - 1) / ew) < 1024) ew /= 2;
+  return ew;
+}
 
 __device__ __forceinline__ double lsq(const double* theta, int nls, int q) {
   return theta[nls == 1 ? 0 : q];
@@ -271,8 +279,8 @@ __global__ __launch_bounds__(256) void gpfrob_kernel(const double* __restrict__ 
 // Kc^T G_P (G_P is symmetric) from Kc = Kzx evaluated once for the chunk.
 // Block (mt, cb): inducing rows mt*TILE .. +TILE (thread row li = t % TILE; the
 // two halves of the block take alternate points) against points
-// c0 + cb*EW .. +EW.  The kernel value and its derivative factor are
-// recomputed from the inputs per element.  Partials, split = c0 / EW + cb:
+// c0 + cb*ew .. +ew.  The kernel value and its derivative factor are
+// recomputed from the inputs per element.  Partials, split = c0 / ew + cb:
 // gzpart[(split * mp + i) * DMAX + q] and
 // tpart[(split * mt_count + mt) * (DMAX + 1) + q] (lengthscales, then variance).
 // Mixed path (TW = float): Wt in float32 and the kernel value and factor in
@@ -281,7 +289,7 @@ template <int DMAX, typename TW>
 __global__ __launch_bounds__(256) void elbo_wgrad_kernel(
     int kind, const double* __restrict__ x, const double* __restrict__ y,
     const double* __restrict__ z, int64_t m, int d, const double* __restrict__ theta, int nls,
-    const TW* __restrict__ Wt, int64_t mp, int64_t c0, int64_t ncol,
+    const TW* __restrict__ Wt, int64_t mp, int64_t c0, int64_t ncol, int64_t ew,
     const double* __restrict__ cvec, double* __restrict__ gzpart, double* __restrict__ tpart) {
   __shared__ double xc[TILE][DMAX + 1];
   __shared__ double rc[TILE];
@@ -302,8 +310,8 @@ __global__ __launch_bounds__(256) void elbo_wgrad_kernel(
   }
   const double gb = rowok ? cvec[gi] / (s * s) : 0.0;
   double s_var = 0.0;
-  const int64_t p0 = c0 + cb * EW;
-  const int64_t p1 = (p0 + EW < c0 + ncol) ? p0 + EW : c0 + ncol;
+  const int64_t p0 = c0 + cb * ew;
+  const int64_t p1 = (p0 + ew < c0 + ncol) ? p0 + ew : c0 + ncol;
   for (int64_t b0 = p0; b0 < p1; b0 += TILE) {
     __syncthreads();
     for (int e = t; e < TILE * DMAX; e += 256) {
@@ -344,7 +352,7 @@ __global__ __launch_bounds__(256) void elbo_wgrad_kernel(
     for (int q = 0; q < DMAX; ++q) gzs[li][q] = gzr[q];
   }
   __syncthreads();
-  const int64_t split = c0 / EW + cb;
+  const int64_t split = c0 / ew + cb;
   if (half == 0) {
 #pragma unroll
     for (int q = 0; q < DMAX; ++q) gzpart[(split * mp + gi) * DMAX + q] = gzr[q] + gzs[li][q];
@@ -362,53 +370,65 @@ __global__ __launch_bounds__(256) void elbo_wgrad_kernel(
         red_s[0][t] + red_s[1][t] + red_s[2][t] + red_s[3][t];
 }
 
-// ---- E4: tr(G_K dKzz) terms; one thread per inducing point (row), G_K symmetric ----
+// ---- E4: tr(G_K dKzz) terms (G_K symmetric) ----
+// Block (rb, cb): inducing rows rb*KZZ_ROWS .. + KZZ_ROWS against the inducing points
+// cb*KZZ_COLS .. + KZZ_COLS; thread (row t % 64, quarter t / 64) takes every fourth
+// point.  Partials per (cb, row) and per block.  (One thread per row over all points,
+// 256 rows per block, left m = 2,048 with eight workgroups: 1,105 us, now 89 us.)
+constexpr int KZZ_ROWS = 64;
+constexpr int KZZ_COLS = 128;
 template <int DMAX>
 __global__ __launch_bounds__(256) void elbo_kzz_adj_kernel(
     int kind, const double* __restrict__ z, int64_t m, int d, const double* __restrict__ theta,
     int nls, const double* __restrict__ GK, int64_t ld, double* __restrict__ gzkz,
     double* __restrict__ tpart) {
-  __shared__ double zj[256][DMAX + 1];
+  __shared__ double zj[KZZ_COLS][DMAX + 1];
+  __shared__ double gzs[3][KZZ_ROWS][DMAX];
   __shared__ double red_s[4][DMAX + 1];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const int64_t i = (int64_t)blockIdx.x * 256 + t;
+  const int64_t i = (int64_t)blockIdx.x * KZZ_ROWS + lane;
+  const int64_t j0 = (int64_t)blockIdx.y * KZZ_COLS;
   double zi[DMAX];
 #pragma unroll
   for (int q = 0; q < DMAX; ++q) zi[q] = (q < d && i < m) ? z[i * d + q] / lsq(theta, nls, q) : 0.0;
+  for (int e = t; e < KZZ_COLS * DMAX; e += 256) {
+    const int r = e / DMAX, q = e % DMAX;
+    const int64_t g = j0 + r;
+    zj[r][q] = (q < d && g < m) ? z[g * d + q] / lsq(theta, nls, q) : 0.0;
+  }
+  __syncthreads();
   double s_var = 0.0, s_ls[DMAX], gzr[DMAX];
 #pragma unroll
   for (int q = 0; q < DMAX; ++q) {
     s_ls[q] = 0.0;
     gzr[q] = 0.0;
   }
-  for (int64_t j0 = 0; j0 < m; j0 += 256) {
-    __syncthreads();
-    for (int e = t; e < 256 * DMAX; e += 256) {
-      const int r = e / DMAX, q = e % DMAX;
-      const int64_t g = j0 + r;
-      zj[r][q] = (q < d && g < m) ? z[g * d + q] / lsq(theta, nls, q) : 0.0;
-    }
-    __syncthreads();
-    if (i < m) {
-      const int64_t jn = (m - j0 < 256) ? m - j0 : 256;
-      for (int jj = 0; jj < jn; ++jj) {
-        const double g = GK[(j0 + jj) * ld + i];
-        double kv, fv;
-        kval_fac(kind, d2_of<DMAX>(zi, zj[jj]), kv, fv);
-        s_var += g * kv;
-        const double gf = g * fv;
+  if (i < m) {
+    const int jn = (m - j0 < KZZ_COLS) ? (int)(m - j0) : KZZ_COLS;
+    for (int jj = w; jj < jn; jj += 4) {
+      const double g = GK[(j0 + jj) * ld + i];
+      double kv, fv;
+      kval_fac(kind, d2_of<DMAX>(zi, zj[jj]), kv, fv);
+      s_var += g * kv;
+      const double gf = g * fv;
 #pragma unroll
-        for (int q = 0; q < DMAX; ++q) {
-          const double df = zi[q] - zj[jj][q];
-          s_ls[q] += gf * df * df;
-          gzr[q] += gf * df;
-        }
+      for (int q = 0; q < DMAX; ++q) {
+        const double df = zi[q] - zj[jj][q];
+        s_ls[q] += gf * df * df;
+        gzr[q] += gf * df;
       }
     }
   }
-  if (i < m) {
+  if (w > 0) {
 #pragma unroll
-    for (int q = 0; q < DMAX; ++q) gzkz[i * DMAX + q] = gzr[q];
+    for (int q = 0; q < DMAX; ++q) gzs[w - 1][lane][q] = gzr[q];
+  }
+  __syncthreads();
+  if (w == 0) {
+#pragma unroll
+    for (int q = 0; q < DMAX; ++q)
+      gzkz[((int64_t)blockIdx.y * ld + i) * DMAX + q] =
+          ((gzr[q] + gzs[0][lane][q]) + gzs[1][lane][q]) + gzs[2][lane][q];
   }
 #pragma unroll
   for (int q = 0; q < DMAX + 1; ++q) {
@@ -419,7 +439,8 @@ __global__ __launch_bounds__(256) void elbo_kzz_adj_kernel(
   }
   __syncthreads();
   if (t < DMAX + 1)
-    tpart[blockIdx.x * (DMAX + 1) + t] = red_s[0][t] + red_s[1][t] + red_s[2][t] + red_s[3][t];
+    tpart[((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * (DMAX + 1) + t] =
+        red_s[0][t] + red_s[1][t] + red_s[2][t] + red_s[3][t];
 }
 
 // ---- scalar slots ----
@@ -455,12 +476,14 @@ __global__ __launch_bounds__(256) void elbo_fwd_finalize(
     for (int k = threadIdx.x; k < nf; k += 256) gp2 += epart[k];
     gp2 = block_sum256(gp2, red);
   }
+  double rr = 0.0, sr = 0.0;
+  for (int k = threadIdx.x; k < nr; k += 256) {
+    rr += rpart[2 * k];
+    sr += rpart[2 * k + 1];
+  }
+  rr = block_sum256(rr, red);
+  sr = block_sum256(sr, red);
   if (threadIdx.x == 0) {
-    double rr = 0.0, sr = 0.0;
-    for (int k = 0; k < nr; ++k) {
-      rr += rpart[2 * k];
-      sr += rpart[2 * k + 1];
-    }
     double ldk = 0.0, ldc = 0.0;
     int info = 0;
     for (int64_t k = 0; k < nleaf; ++k) {
@@ -529,7 +552,7 @@ __global__ __launch_bounds__(256) void elbo_bwd_scalars(const double* __restrict
 __global__ __launch_bounds__(256) void elbo_grad_finalize(
     const double* __restrict__ tpart, int64_t nt3, const double* __restrict__ tpart2,
     int64_t nt4, const double* __restrict__ gzpart, int64_t S2, const double* __restrict__ gzkz,
-    const double* __restrict__ c, const double* __restrict__ qv, const double* __restrict__ scal,
+    int64_t nkz, const double* __restrict__ c, const double* __restrict__ qv, const double* __restrict__ scal,
     int64_t m, int64_t mp, int d, int64_t n, const double* __restrict__ theta, int nls,
     double gbar, double* __restrict__ grad, double* __restrict__ grad_z, int dmax) {
   __shared__ double red[4];
@@ -570,18 +593,34 @@ __global__ __launch_bounds__(256) void elbo_grad_finalize(
     }
     return;
   }
-  const int64_t e = (int64_t)(q - (nls + 3)) * 256 + threadIdx.x;
-  if (e >= m * d) return;
-  const int64_t i = e / d;
-  const int qq = (int)(e % d);
-  double g = gzkz[i * dmax + qq];
-  for (int64_t k = 0; k < S2; ++k) g += gzpart[(k * mp + i) * dmax + qq];
-  grad_z[e] = gbar * (-var * g / lsq(theta, nls, qq));
+  // g_Z: 64 entries per block; its four waves take every fourth partial, four of
+  // them in flight, and their sums are added in wave order
+  __shared__ double gsum[4][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int64_t e = (int64_t)(q - (nls + 3)) * 64 + lane;
+  const bool ok = e < m * d;
+  const int64_t i = ok ? e / d : 0;
+  const int qq = ok ? (int)(e % d) : 0;
+  double g[4] = {0.0, 0.0, 0.0, 0.0};
+  const double* src = gzpart + i * dmax + qq;
+  int64_t k = w;
+  for (; k + 12 < S2; k += 16) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) g[u] += src[(k + 4 * u) * mp * dmax];
+  }
+  for (; k < S2; k += 4) g[0] += src[k * mp * dmax];
+  for (k = w; k < nkz; k += 4) g[1] += gzkz[(k * mp + i) * dmax + qq];
+  gsum[w][lane] = (g[0] + g[1]) + (g[2] + g[3]);
+  __syncthreads();
+  if (w == 0 && ok)
+    grad_z[e] = gbar * (-var * (((gsum[0][lane] + gsum[1][lane]) + gsum[2][lane]) + gsum[3][lane]) /
+                        lsq(theta, nls, qq));
 }
 
 // ---- workspace layout ----
 struct ElboLayout {
-  int64_t mp = 0, mt = 0, ntile = 0, S2 = 1, chunk2 = EW, nbw = TILE;
+  int64_t mp = 0, mt = 0, ntile = 0, S2 = 1, ew = 1024, nbw = TILE;
+  int64_t kz64 = TILE, nbw64 = TILE, nkz = 1;
   int64_t nr = 256, nf = 1024;
   size_t off_K = 0, off_XK = 0, off_C = 0, off_XC = 0, off_P = 0, off_Kinv = 0, off_Cinv = 0;
   size_t off_G = 0, off_T1 = 0, off_T2 = 0, off_T = 0;
@@ -598,6 +637,18 @@ struct ElboLayout {
 
 inline size_t al(size_t b) { return (b + 255) / 256 * 256; }
 
+// Columns per split of the float64 statistics product P = Kc Kc^T (lower tiles, K =
+// the chunk's columns): 1,024, or fewer (down to 256) until the launch has 512
+// workgroups, and at least mp, which keeps the splits' partials apart within a row
+// of the buffer.  The chunk is padded with zero columns to a whole number of splits.
+// (Halving the chunk while its width stayed a multiple of 128 left a 50,048-column
+// chunk, 391 tiles wide, in one split: 6.7 ms on 10 workgroups, now 297 us.)
+int64_t split_columns(int64_t nbw, int64_t mp, int64_t ntile) {
+  int64_t kz = 1024;
+  while (kz > 256 && ntile * ((nbw + kz - 1) / kz) < 512) kz /= 2;
+  return kz < mp ? mp : kz;
+}
+
 ElboLayout make_elbo_layout(int64_t n, int64_t m) {
   ElboLayout L;
   L.mp = round_up(m, 256);
@@ -607,8 +658,11 @@ ElboLayout make_elbo_layout(int64_t n, int64_t m) {
   // forward's split-K partials of P are mp columns wide within a row of nbw)
   L.nbw = round_up(n, TILE) < BW_CHUNK ? round_up(n, TILE) : BW_CHUNK;
   if (L.nbw < L.mp) L.nbw = L.mp;
-  L.chunk2 = EW;
-  L.S2 = (n + EW - 1) / EW;
+  L.ew = wgrad_points(n, L.mt);
+  L.S2 = (n + L.ew - 1) / L.ew;
+  L.kz64 = split_columns(L.nbw, L.mp, L.ntile);
+  L.nbw64 = round_up(L.nbw, L.kz64);
+  L.nkz = (L.mp + KZZ_COLS - 1) / KZZ_COLS;
   const int64_t mp = L.mp;
   const size_t M2 = (size_t)mp * mp * sizeof(double);
   const size_t V = (size_t)mp * sizeof(double);
@@ -638,16 +692,16 @@ ElboLayout make_elbo_layout(int64_t n, int64_t m) {
   L.off_Pc = o; o += al(V);
   L.off_gzpart = o; o += al((size_t)L.S2 * mp * EDMAX * sizeof(double));
   L.off_tpart = o; o += al((size_t)L.S2 * L.mt * (EDMAX + 1) * sizeof(double));
-  L.off_tpart2 = o; o += al((size_t)(mp / 256) * (EDMAX + 1) * sizeof(double));
-  L.off_gzkz = o; o += al((size_t)mp * EDMAX * sizeof(double));
+  L.off_tpart2 = o; o += al((size_t)(mp / KZZ_ROWS) * L.nkz * (EDMAX + 1) * sizeof(double));
+  L.off_gzkz = o; o += al((size_t)L.nkz * mp * EDMAX * sizeof(double));
   L.off_rpart = o; o += al((size_t)L.nr * 2 * sizeof(double));
   L.off_fpart = o; o += al((size_t)L.nf * sizeof(double));
   L.off_epart = o; o += al((size_t)L.nf * sizeof(double));
   L.off_fs = o; o += al(4 * sizeof(float));
   L.off_vpart = o; o += al((size_t)((mp + 1023) / 1024) * mp * sizeof(double));
   L.off_scal = o; o += al(32 * sizeof(double));
-  L.off_kc = o; o += al((size_t)mp * L.nbw * sizeof(double));
-  L.off_wt = o; o += al((size_t)L.nbw * mp * sizeof(double));
+  L.off_kc = o; o += al((size_t)mp * L.nbw64 * sizeof(double));
+  L.off_wt = o; o += al((size_t)L.nbw64 * mp * sizeof(double));
   L.total = o;
   return L;
 }
@@ -723,21 +777,27 @@ int elbo_forward_impl(int kind, const ElboArith& ea, const double* x, const doub
   //    entry) bytes): member z reads columns z*kz .. +kz of Kc and accumulates
   //    its float64 partial of P at column z*kp (kp = kz for float64 chunks,
   //    kz / 2 for float32 ones; kp >= mp keeps the partials apart) of a
-  //    [mp][nbw] float64 buffer (the one that holds Wt in the backward).  S is
-  //    the largest power of two up to 64 that keeps kp >= mp: at M = 2,048
-  //    and 131,072-point chunks, S = 32 (float32 chunks, 4,352 workgroups, one
+  //    [mp][nbw] float64 buffer (the one that holds Wt in the backward).  Float64:
+  //    split_columns.  Float32: S is the largest power of two up to 64 that keeps
+  //    kp >= mp (the correction products' fp32 chains run over a member's whole
+  //    k-range, so there S is part of the arithmetic).  At M = 2,048 and
+  //    131,072-point chunks, S = 32 (float32 chunks, 4,352 workgroups, one
   //    resident per CU) or S = 64 (float64, 8,704, two per CU), 17 full rounds
-  //    of the chip either way (65,536-point chunks left half a round idle).
+  //    of the chip either way (65,536-point chunks left half a round idle).  A
+  //    chunk shorter than nbw runs only the members that hold points of it.
   const size_t ke = ea.f32 ? sizeof(float) : sizeof(double);
   double* Pp = at<double>(ws, Lo.off_wt);
-  const int64_t nbw = Lo.nbw;
   const int64_t kdiv = ea.f32 ? 2 : 1;
-  int64_t S = 1;
-  while (S < 64 && (nbw / (2 * S)) % TILE == 0 && nbw / (2 * S) >= kdiv * mp) S *= 2;
+  int64_t nbw = Lo.nbw, S = 1;
+  if (ea.f32) {
+    while (S < 64 && (nbw / (2 * S)) % TILE == 0 && nbw / (2 * S) >= kdiv * mp) S *= 2;
+  } else {
+    nbw = Lo.nbw64;
+    S = nbw / Lo.kz64;
+  }
   const int64_t kz = nbw / S, kp = kz / kdiv;
   Batch sk;
   sk.ws_stride = kz * (int64_t)ke;
-  sk.count = (unsigned)S;
   float* fs = at<float>(ws, Lo.off_fs);
   if (ea.f32 && ea.fwd == AR_FP16X3) {
     hipLaunchKernelGGL(elbo_fp16_scale_kernel, dim3(1), dim3(64), 0, s, theta, nls, nullptr, 0,
@@ -775,10 +835,12 @@ int elbo_forward_impl(int kind, const ElboArith& ea, const double* x, const doub
     FK.s = s;
     for (int64_t c0 = 0; c0 < n; c0 += BW_CHUNK) {
       const int64_t ncol = (n - c0 < BW_CHUNK) ? n - c0 : BW_CHUNK;
+      sk.count = (unsigned)((ncol + kz - 1) / kz);
+      const int64_t ncolp = sk.count * kz;
       if (ea.f32) {
         float* Kc = at<float>(ws, Lo.off_kc);
         GPK_TRY(launch_cross<float>(kind, z, m, x + c0 * d, ncol, d, theta, nls, true, Kc, nbw,
-                                    mp, nbw, s));
+                                    mp, ncolp, s));
         GPK_TRY(launch_gemm<float, float, double>(ea.fwd, false, false, Kc, nbw, Kc, nbw, Pp, nbw,
                                                   mp, mp, kz, 1.0, c0 > 0, true, KR_FULL, s,
                                                   nullptr, sk, fs));
@@ -787,7 +849,7 @@ int elbo_forward_impl(int kind, const ElboArith& ea, const double* x, const doub
       } else {
         double* Kc = at<double>(ws, Lo.off_kc);
         GPK_TRY(launch_cross<double>(kind, z, m, x + c0 * d, ncol, d, theta, nls, false, Kc, nbw,
-                                     mp, nbw, s));
+                                     mp, ncolp, s));
         GPK_TRY(launch_gemm<double, double, double>(AR_F64, false, false, Kc, nbw, Kc, nbw, Pp,
                                                     nbw, mp, mp, kz, 1.0, c0 > 0, true, KR_FULL, s,
                                                     nullptr, sk));
@@ -898,7 +960,8 @@ int elbo_backward_impl(int kind, const ElboArith& ea, const double* x, const dou
                        cvec, mp, mp, theta, nls);
     GPK_LAUNCH_CHECK();
 #define GPK_E4(DM)                                                                              \
-  hipLaunchKernelGGL(elbo_kzz_adj_kernel<DM>, dim3((unsigned)(mp / 256)), dim3(256), 0, s2, kind, \
+  hipLaunchKernelGGL(elbo_kzz_adj_kernel<DM>, dim3((unsigned)(mp / KZZ_ROWS), (unsigned)Lo.nkz), \
+                     dim3(256), 0, s2, kind,                                                    \
                      z, m, d, theta, nls, T1, mp, at<double>(ws, Lo.off_gzkz),                   \
                      at<double>(ws, Lo.off_tpart2))
     GPK_DMAX_DISPATCH(d, GPK_E4);
@@ -943,16 +1006,16 @@ int elbo_backward_impl(int kind, const ElboArith& ea, const double* x, const dou
         GPK_TRY(launch_gemm<double, double, double>(AR_F64, true, false, Kc, ncp, G, mp, Wt, mp,
                                                     ncp, mp, mp, 1.0, false, false, KR_FULL, s));
       }
-      dim3 grid((unsigned)Lo.mt, (unsigned)((ncol + EW - 1) / EW));
+      dim3 grid((unsigned)Lo.mt, (unsigned)((ncol + Lo.ew - 1) / Lo.ew));
 #define GPK_E3(DM)                                                                         \
   do {                                                                                     \
     if (ea.f32)                                                                            \
       hipLaunchKernelGGL((elbo_wgrad_kernel<DM, float>), grid, dim3(256), 0, s, kind, x, y, \
-                         z, m, d, theta, nls, Wtf, mp, c0, ncol, cvec,                     \
+                         z, m, d, theta, nls, Wtf, mp, c0, ncol, Lo.ew, cvec,              \
                          at<double>(ws, Lo.off_gzpart), at<double>(ws, Lo.off_tpart));     \
     else                                                                                   \
       hipLaunchKernelGGL((elbo_wgrad_kernel<DM, double>), grid, dim3(256), 0, s, kind, x,  \
-                         y, z, m, d, theta, nls, Wt, mp, c0, ncol, cvec,                   \
+                         y, z, m, d, theta, nls, Wt, mp, c0, ncol, Lo.ew, cvec,            \
                          at<double>(ws, Lo.off_gzpart), at<double>(ws, Lo.off_tpart));     \
   } while (0)
       GPK_DMAX_DISPATCH(d, GPK_E3);
@@ -966,11 +1029,11 @@ int elbo_backward_impl(int kind, const ElboArith& ea, const double* x, const dou
   else if (d <= 4) dmax = 4;
   else if (d <= 8) dmax = 8;
   else if (d <= 16) dmax = 16;
-  const unsigned gblocks = (unsigned)(nls + 3) + cdiv(m * d, 256);
+  const unsigned gblocks = (unsigned)(nls + 3) + cdiv(m * d, 64);
   hipLaunchKernelGGL(elbo_grad_finalize, dim3(gblocks), dim3(256), 0, s,
                      at<double>(ws, Lo.off_tpart), Lo.S2 * Lo.mt, at<double>(ws, Lo.off_tpart2),
-                     (int64_t)(mp / 256), at<double>(ws, Lo.off_gzpart), Lo.S2,
-                     at<double>(ws, Lo.off_gzkz), cvec, at<double>(ws, Lo.off_q), scal, m, mp, d,
+                     (int64_t)(mp / KZZ_ROWS) * Lo.nkz, at<double>(ws, Lo.off_gzpart), Lo.S2,
+                     at<double>(ws, Lo.off_gzkz), Lo.nkz, cvec, at<double>(ws, Lo.off_q), scal, m, mp, d,
                      n, theta, nls, gbar, grad, grad_z, dmax);
   GPK_LAUNCH_CHECK();
   return GPK_OK;
