@@ -124,7 +124,7 @@ struct Layout {
   // r, alpha, u and v each lead a block of nvec vectors (np apart): with the
   // mixed path's probes, [r z1 z2], [alpha w1 w2], [u u1 u2], [v v1 v2].
   int nvec = 1;
-  size_t off_r = 0, off_alpha = 0, off_u = 0, off_v = 0, off_res = 0, off_delta = 0;
+  size_t off_r = 0, off_alpha = 0, off_u = 0, off_v = 0, off_res = 0;
   size_t off_skip = 0;
   size_t off_dblk = 0;
   // float32 storage: Sigma's lower NB-tiles in float64, packed, and the
@@ -144,9 +144,10 @@ Layout make_layout(int64_t n, int64_t d, int prec, int spk = -1) {
   const int64_t np = L.np;
   const int64_t nleaf = np / NB;
   const int64_t ntile = nleaf * (nleaf + 1) / 2;
-  // partial sums of the triangular matvecs (1,024-row chunks) and of the
-  // recomputed Sigma products
-  const int64_t nchunk = std::max((np + 1023) / 1024, sigma_mv_max_chunks(np));
+  // partial sums of the triangular matvecs, of the recomputed Sigma products and of
+  // the column reductions
+  const int64_t nchunk =
+      std::max({trmv_max_chunks(np), sigma_mv_max_chunks(np), colreduce_chunks(np)});
   size_t o = 0;
   L.off_L = o; o += al((size_t)np * np * L.ts);
   L.off_X = o; o += al((size_t)np * np * L.ts);
@@ -161,7 +162,6 @@ Layout make_layout(int64_t n, int64_t d, int prec, int spk = -1) {
   L.off_u = o; o += VB;
   L.off_v = o; o += VB;
   L.off_res = o; o += al((size_t)np * sizeof(double));
-  L.off_delta = o; o += al((size_t)np * sizeof(double));
   L.off_dblk = o; o += al(prec == GPK_PREC_FP64 ? 0 : (size_t)np * NB * sizeof(double));
   L.off_spk = o; o += al(L.has_spk ? (size_t)ntile * NB * NB * sizeof(double) : 0);
   L.off_spart = o;
@@ -176,8 +176,12 @@ Layout make_layout(int64_t n, int64_t d, int prec, int spk = -1) {
 }
 
 // ---- small kernels ----
+// r = y - c on the padded vector; also clears the member's refinement stop flag (a
+// kernel's store, not a memset, so that the forward stays capturable).
 __global__ void prep_r_kernel(const double* __restrict__ y, const double* __restrict__ theta,
-                              int nls, int64_t n, int64_t np, double* __restrict__ r, Batch bt) {
+                              int nls, int64_t n, int64_t np, double* __restrict__ r, int* skip,
+                              Batch bt) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *bws(skip, bt) = 0;
   if (bt.gp) {
     const int64_t p = bt.gp[blockIdx.z];
     y += bt.xoff[p];
@@ -187,31 +191,6 @@ __global__ void prep_r_kernel(const double* __restrict__ y, const double* __rest
   r = bws(r, bt);
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < np) r[i] = i < n ? y[i] - theta[nls + 2] : 0.0;
-}
-
-__global__ void sub_kernel(const double* __restrict__ a, const double* __restrict__ b,
-                           int64_t np, double* __restrict__ out, Batch bt) {
-  if (bskip(bt)) return;
-  a = bws(a, bt);
-  b = bws(b, bt);
-  out = bws(out, bt);
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < np) out[i] = a[i] - b[i];
-}
-
-__global__ void add_kernel(double* __restrict__ a, const double* __restrict__ b, int64_t np,
-                           Batch bt) {
-  if (bskip(bt)) return;
-  a = bws(a, bt);
-  b = bws(b, bt);
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < np) a[i] += b[i];
-}
-
-// Refinement stop flag of each member: cleared at the start of a forward (a
-// kernel, not a memset, so that the forward stays capturable).
-__global__ void skip_clear_kernel(int* skip, Batch bt) {
-  if (threadIdx.x == 0) *bws(skip, bt) = 0;
 }
 
 __device__ double block_sum(double v, double* red);
@@ -529,7 +508,6 @@ int mll_forward_t(int kind, const Arith3& ar, const double* x, const double* y, 
   double* u = at<double>(ws, Lo.off_u);
   double* v = at<double>(ws, Lo.off_v);
   double* res = at<double>(ws, Lo.off_res);
-  double* delta = at<double>(ws, Lo.off_delta);
   double* part = at<double>(ws, Lo.off_part);
   const bool f64 = std::is_same<TS, double>::value;
   Factor<TS> F{L,
@@ -549,10 +527,13 @@ int mll_forward_t(int kind, const Arith3& ar, const double* x, const double* y, 
   double* spk = (Lo.has_spk && vr.stored_sigma) ? at<double>(ws, Lo.off_spk) : nullptr;
   // v = Sigma a (nvv vectors): read from the float64 copy when there is one,
   // otherwise recomputed from the inputs in float64
+  // (and res = r - Sigma alpha with it)
   auto sigma_mv = [&](const Batch& b, int nvv) -> int {
     if (spk)
-      return launch_packed_symv(spk, np, alpha, v, at<double>(ws, Lo.off_spart), s, b, nvv);
-    return launch_sigma_matvec(kind, x, n, np, d, theta, nls, jitter, alpha, v, part, s, b, nvv);
+      return launch_packed_symv(spk, np, alpha, v, at<double>(ws, Lo.off_spart), s, b, nvv, r,
+                                res);
+    return launch_sigma_matvec(kind, x, n, np, d, theta, nls, jitter, alpha, v, part, s, b, nvv, r,
+                               res);
   };
   F.dblk = dblk;
   F.bt = bt;
@@ -563,7 +544,8 @@ int mll_forward_t(int kind, const Arith3& ar, const double* x, const double* y, 
     F.fscale = fs;
   }
 
-  hipLaunchKernelGGL(prep_r_kernel, gv, dim3(256), 0, s, y, theta, nls, n, np, r, bt);
+  int* skip = at<int>(ws, Lo.off_skip);
+  hipLaunchKernelGGL(prep_r_kernel, gv, dim3(256), 0, s, y, theta, nls, n, np, r, skip, bt);
   GPK_LAUNCH_CHECK();
   const bool probes = !f64;
   if (probes) {
@@ -573,9 +555,6 @@ int mll_forward_t(int kind, const Arith3& ar, const double* x, const double* y, 
       GPK_LAUNCH_CHECK();
     }
   }
-  int* skip = at<int>(ws, Lo.off_skip);
-  hipLaunchKernelGGL(skip_clear_kernel, dim3(1, 1, bt.count), dim3(64), 0, s, skip, bt);
-  GPK_LAUNCH_CHECK();
   Batch bts = bt;  // the refinement's launches, which stop once it has converged
   bts.skip = skip;
   {
@@ -604,17 +583,13 @@ int mll_forward_t(int kind, const Arith3& ar, const double* x, const double* y, 
   // 1e-12 ||r|| or `iters` steps; the first Sigma product also forms Sigma w_p.
   for (int it = 0; it < iters; ++it) {
     GPK_TRY(sigma_mv(it == 0 ? bt : bts, it == 0 ? nv : 1));
-    hipLaunchKernelGGL(sub_kernel, gv, dim3(256), 0, s, r, v, np, res, bts);
-    GPK_LAUNCH_CHECK();
     if (it > 0) {
       hipLaunchKernelGGL(refine_check_kernel, dim3(1, 1, bt.count), dim3(256), 0, s, r, res, np,
                          skip, bts);
       GPK_LAUNCH_CHECK();
     }
     GPK_TRY(launch_trmv<TS>(X, np, np, res, u, false, part, s, bts));
-    GPK_TRY(launch_trmv<TS>(X, np, np, u, delta, true, part, s, bts));
-    hipLaunchKernelGGL(add_kernel, gv, dim3(256), 0, s, alpha, delta, np, bts);
-    GPK_LAUNCH_CHECK();
+    GPK_TRY(launch_trmv<TS>(X, np, np, u, alpha, true, part, s, bts, 1, true));
   }
   if (probes && iters == 0) {
     GPK_TRY(sigma_mv(bt, nv));
@@ -633,8 +608,6 @@ int mll_forward_t(int kind, const Arith3& ar, const double* x, const double* y, 
   // in `res` already (alpha has not changed since), so these launches return
   // at once then; otherwise they measure the last correction.
   GPK_TRY(sigma_mv(bts, 1));
-  hipLaunchKernelGGL(sub_kernel, gv, dim3(256), 0, s, r, v, np, res, bts);
-  GPK_LAUNCH_CHECK();
   hipLaunchKernelGGL(finalize_fwd_kernel, dim3(1, 1, bt.count), dim3(256), 0, s,
                      at<double>(ws, Lo.off_leafld), at<int>(ws, Lo.off_leafinfo), np / NB, r,
                      alpha, res, n, np, result, bt);
@@ -710,7 +683,7 @@ PredLayout make_pred_layout(const Layout& Lo, int64_t t, int full_cov) {
   P.off_kxt = o; o += al((size_t)np * tc * sizeof(double));
   P.off_a = o; o += al((size_t)np * tc * sizeof(double));
   P.off_ktt = o; o += al((size_t)(full_cov ? tp * tp : 1) * sizeof(double));
-  P.off_part = o; o += al((size_t)((np + 1023) / 1024) * tc * sizeof(double));
+  P.off_part = o; o += al((size_t)colreduce_chunks(np) * tc * sizeof(double));
   P.off_vec = o; o += al((size_t)tc * sizeof(double));
   P.off_res = o; o += al((size_t)GPK_RESULT_LEN * sizeof(double));
   P.total = o;

@@ -698,7 +698,9 @@ ElboLayout make_elbo_layout(int64_t n, int64_t m) {
   L.off_fpart = o; o += al((size_t)L.nf * sizeof(double));
   L.off_epart = o; o += al((size_t)L.nf * sizeof(double));
   L.off_fs = o; o += al(4 * sizeof(float));
-  L.off_vpart = o; o += al((size_t)((mp + 1023) / 1024) * mp * sizeof(double));
+  const int64_t nvec = trmv_max_chunks(mp) > colreduce_chunks(mp) ? trmv_max_chunks(mp)
+                                                                  : colreduce_chunks(mp);
+  L.off_vpart = o; o += al((size_t)nvec * mp * sizeof(double));
   L.off_scal = o; o += al(32 * sizeof(double));
   L.off_kc = o; o += al((size_t)mp * L.nbw64 * sizeof(double));
   L.off_wt = o; o += al((size_t)L.nbw64 * mp * sizeof(double));
@@ -1105,7 +1107,7 @@ ElboPredLayout make_elbo_pred_layout(const ElboLayout& Lo, int64_t t, int full_c
   P.off_a1 = o; o += al((size_t)mp * tc * sizeof(double));
   P.off_a2 = o; o += al((size_t)mp * tc * sizeof(double));
   P.off_ktt = o; o += al((size_t)(full_cov ? tp * tp : 1) * sizeof(double));
-  P.off_part = o; o += al((size_t)((mp + 1023) / 1024) * tc * sizeof(double));
+  P.off_part = o; o += al((size_t)colreduce_chunks(mp) * tc * sizeof(double));
   P.off_v1 = o; o += al((size_t)tc * sizeof(double));
   P.off_v2 = o; o += al((size_t)tc * sizeof(double));
   P.off_res = o; o += al(GPK_RESULT_LEN * sizeof(double));

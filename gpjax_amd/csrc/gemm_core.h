@@ -157,13 +157,14 @@ constexpr size_t smem_bytes() {
 
 // One 16-deep k-slab of FP64 matrix-core products from LDS operands stored
 // k-major: a[k * ldp + m], b[k * ldp + n]; the wave owns rows wm*64 .. +64 and
-// columns wn*16*NJ .. +16*NJ.
+// columns wn*16*NJ .. +16*NJ.  Product kk takes k = kk, 4 + kk, 8 + kk, 12 + kk, as
+// the small-tile kernels do (gemm.hip), so all tile widths give the same bits.
 template <int NJ = 4>
 __device__ __forceinline__ void mfma_slab_f64(const double* a, const double* b, int ldp,
                                               int lane, int wm, int wn, f64x4 (&acc)[4][NJ]) {
 #pragma unroll
   for (int kk = 0; kk < 4; ++kk) {
-    const int kr = kk * 4 + (lane >> 4);
+    const int kr = kk + 4 * (lane >> 4);
     double av[4], bv[NJ];
 #pragma unroll
     for (int i = 0; i < 4; ++i) av[i] = a[kr * ldp + wm * 64 + i * 16 + (lane & 15)];

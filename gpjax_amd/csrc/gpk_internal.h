@@ -241,7 +241,8 @@ enum KRange { KR_FULL = 0, KR_GE_N = 1, KR_LE_M = 2, KR_GE_M = 3 };
 enum Arith { AR_F64 = 0, AR_BF16X3 = 3, AR_FP16X3 = 4, AR_BF16X6 = 6 };
 
 // Tile rule of the FP64 products (double operands, no diagonal side buffer), by the
-// number of 128-tiles of the launch: up to SMALL_TILES run on 64 x 64 tiles, up to
+// number of 128-tiles of the launch (every tile width sums k in the same order, so
+// the choice changes no bit): up to SMALL_TILES run on 64 x 64 tiles, up to
 // TINY_TILES on 32 x 32.  The line lies where 128-tiles fill the chip's two
 // workgroups per CU; MLL + gradient at n = 5,000: 6.57 ms with 160, 6.45 with 384,
 // 6.19 with 512, 6.27 with 1,024 (10.9 without), n = 16,384: 86.5 / 86.8 / 86.7 /
@@ -330,13 +331,35 @@ template <typename TS>
 int launch_lower_to_upper(const TS* X, TS* U, int64_t ld, int64_t np, hipStream_t s,
                           const Batch& bt = Batch());
 
-// y = X r (trans = false) or y = X^T r (trans = true), X lower triangular
-// np x np (only k <= i is read); float64 accumulation through `partial`
-// (nv x ceil(np / 1024) x np doubles).  nv = 1 or 3 right-hand sides, stored
+// Row chunk of launch_trmv's transposed form over its 64-column blocks: the widest of
+// 1,024 .. 128 rows whose grid (column blocks x chunks x members) has at least 1,024
+// workgroups, 128 if none has; and the most chunks it makes of np rows.
+inline int64_t trmv_t_rows(int64_t np, int64_t members) {
+  const int64_t blocks = (np + 63) / 64;
+  int64_t rc = 1024;
+  while (rc > 128 && blocks * ((np + rc - 1) / rc) * members < 1024) rc /= 2;
+  return rc;
+}
+inline int64_t trmv_max_chunks(int64_t np) {
+  const int64_t rc = trmv_t_rows(np, 1);
+  return (np + rc - 1) / rc;
+}
+// Row chunk of launch_colreduce, by the number of rows alone: a column's sum does not
+// depend on how many columns come with it (the predictive's passes).
+inline int64_t colreduce_rows(int64_t rows) { return rows <= 4096 ? 128 : rows <= 16384 ? 256 : 1024; }
+inline int64_t colreduce_chunks(int64_t rows) {
+  const int64_t rc = colreduce_rows(rows);
+  return (rows + rc - 1) / rc;
+}
+
+// y = X r (trans = false) or y = X^T r (trans = true; add: y += X^T r), X lower
+// triangular np x np (only k <= i is read); float64 accumulation through `partial`
+// (nv x trmv_max_chunks(np) x np doubles).  nv = 1 or 3 right-hand sides, stored
 // np apart in r and in y, share each pass over X.
 template <typename TS>
 int launch_trmv(const TS* X, int64_t ld, int64_t np, const double* r, double* y, bool trans,
-                double* partial, hipStream_t s, const Batch& bt = Batch(), int nv = 1);
+                double* partial, hipStream_t s, const Batch& bt = Batch(), int nv = 1,
+                bool add = false);
 
 // Columns per chunk of the recomputed Sigma product below: the widest power of two
 // (64 .. 1,024) whose grid, ceil(np / 256) row blocks x chunks x members, has at
@@ -355,10 +378,11 @@ inline int64_t sigma_mv_max_chunks(int64_t np) {
 
 // v = Sigma a, Sigma recomputed from x in float64 (identity pad for i >= n);
 // nv = 1 or 3 vectors np apart share each kernel evaluation.  partial holds
-// nv x sigma_mv_max_chunks(np) x np doubles.
+// nv x sigma_mv_max_chunks(np) x np doubles.  res (optional) = r - v (first vector).
 int launch_sigma_matvec(int kind, const double* x, int64_t n, int64_t np, int d,
                         const double* theta, int nls, double jitter, const double* a, double* v,
-                        double* partial, hipStream_t s, const Batch& bt = Batch(), int nv = 1);
+                        double* partial, hipStream_t s, const Batch& bt = Batch(), int nv = 1,
+                        const double* r = nullptr, double* res = nullptr);
 
 // Library-owned streams (default priority, non-blocking) and events for the
 // calling thread on the current device, created on first use and kept for the
@@ -385,12 +409,14 @@ struct StreamJoin {
 // v = S a for a symmetric S held as its packed lower NB-tiles in float64 (the
 // spk layout of launch_kernel_matrix), np x np; nv = 1 or 3 vectors np apart
 // share each read of S.  partial holds 2 * nv * T(T+1)/2 * NB doubles, T = np/NB.
+// res (optional) = r - v (first vector).
 int launch_packed_symv(const double* S, int64_t np, const double* a, double* v,
-                       double* partial, hipStream_t s, const Batch& bt = Batch(), int nv = 1);
+                       double* partial, hipStream_t s, const Batch& bt = Batch(), int nv = 1,
+                       const double* r = nullptr, double* res = nullptr);
 
 // y_j = sum_i M[i][j] v_i (v non-null) or sum_i M[i][j]^2 (v null), dense
 // rows x cols (float64 or float32 entries, float64 sums); partial holds
-// ceil(rows/1024) x cols doubles.  lower: only rows i >= j enter column j.
+// colreduce_chunks(rows) x cols doubles.  lower: only rows i >= j enter column j.
 template <typename TM>
 int launch_colreduce(const TM* M, int64_t ld, int64_t rows, int64_t cols, const double* v,
                      double* y, double* partial, hipStream_t s, bool lower = false);

@@ -45,7 +45,7 @@ LinLayout make_lin_layout(int64_t n, int64_t m, int prec) {
   P.off_C = o; o += al256((size_t)np * P.mp * sizeof(double));
   P.off_r = o; o += al256((size_t)np * sizeof(double));
   P.off_u = o; o += al256((size_t)np * sizeof(double));
-  P.off_part = o; o += al256((size_t)((np + 1023) / 1024) * np * sizeof(double));
+  P.off_part = o; o += al256((size_t)trmv_max_chunks(np) * np * sizeof(double));
   P.off_scal = o; o += al256(4 * sizeof(double));
   P.total = o;
   return P;

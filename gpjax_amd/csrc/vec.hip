@@ -9,13 +9,15 @@ namespace gpk {
 namespace {
 
 constexpr int TRMV_CW = 2048;  // columns per chunk, non-transposed
-constexpr int TRMV_RC = 1024;  // rows per chunk, transposed
+constexpr int TRMV_RC = 1024;  // most rows per chunk, transposed
 
-// y_i partial over columns [c*CW, (c+1)*CW), k <= i.  One wave per row, 16 rows
-// per workgroup; each lane reads 16 bytes per load (four float32 or two
-// float64 entries, 1 KB per wave), the row's tail up to the diagonal entry by
-// entry.  NV right-hand sides (stride np) share every load of X.
-template <typename TS, int NV>
+// y_i partial over columns [c*CW, (c+1)*CW), k <= i.  One wave per row, RW rows per
+// wave; each lane reads 16 bytes per load (four float32 or two float64 entries,
+// 1 KB per wave), the row's tail up to the diagonal entry by entry.  NV right-hand
+// sides (stride np) share every load of X.  RW = 4 shares the staged right-hand side
+// between 16 rows; RW = 1 is for grids that would leave most of the chip idle
+// (np = 2,048: 23 -> 9 us).
+template <typename TS, int NV, int RW>
 __global__ __launch_bounds__(256) void trmv_n_kernel(const TS* __restrict__ X, int64_t ld,
                                                      int64_t np, const double* __restrict__ r,
                                                      double* __restrict__ partial, Batch bt) {
@@ -25,19 +27,20 @@ __global__ __launch_bounds__(256) void trmv_n_kernel(const TS* __restrict__ X, i
   partial = bws(partial, bt);
   const int64_t c = blockIdx.y;
   const int64_t nc = gridDim.y;
-  const int64_t row0 = (int64_t)blockIdx.x * 16;
+  const int64_t row0 = (int64_t)blockIdx.x * 4 * RW;
   const int64_t k0 = c * TRMV_CW;
-  if (k0 > row0 + 15) return;
+  if (k0 > row0 + 4 * RW - 1) return;
   __shared__ double rs[NV][TRMV_CW];
-  for (int e = threadIdx.x; e < TRMV_CW; e += 256)
+  const int64_t rend = row0 + 4 * RW - k0;  // columns past the last row's diagonal are not read
+  for (int e = threadIdx.x; e < TRMV_CW && e < rend; e += 256)
 #pragma unroll
     for (int q = 0; q < NV; ++q) rs[q][e] = (k0 + e < np) ? r[q * np + k0 + e] : 0.0;
   __syncthreads();
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   constexpr int V = 16 / sizeof(TS);  // entries per 16-byte load
   typedef typename std::conditional<sizeof(TS) == 4, float4, double2>::type Vec;
-  for (int qr = 0; qr < 4; ++qr) {
-    const int64_t i = row0 + w * 4 + qr;
+  for (int qr = 0; qr < RW; ++qr) {
+    const int64_t i = row0 + w * RW + qr;
     const int64_t kend = (i + 1 < k0 + TRMV_CW) ? i + 1 : k0 + TRMV_CW;
     double acc[NV];
 #pragma unroll
@@ -83,7 +86,7 @@ __global__ void trmv_n_reduce(const double* __restrict__ partial, int64_t np, in
   }
 }
 
-// y_k partial over rows [c*RC, (c+1)*RC), i >= k.  64 columns per workgroup;
+// y_k partial over rows [c*rc, (c+1)*rc), i >= k.  64 columns per workgroup;
 // its four waves take every fourth row (each wave reads 64 consecutive
 // columns of a row, 512 or 256 bytes), so four times as many row loads are in
 // flight per column, and the four row sums are added in a fixed order.  NV
@@ -91,7 +94,8 @@ __global__ void trmv_n_reduce(const double* __restrict__ partial, int64_t np, in
 constexpr int TRMV_TC = 64;  // columns per workgroup, transposed
 template <typename TS, int NV>
 __global__ __launch_bounds__(256) void trmv_t_kernel(const TS* __restrict__ X, int64_t ld,
-                                                     int64_t np, const double* __restrict__ r,
+                                                     int64_t np, int64_t rc,
+                                                     const double* __restrict__ r,
                                                      double* __restrict__ partial, Batch bt) {
   if (bskip(bt)) return;
   X = bws(X, bt);
@@ -100,12 +104,12 @@ __global__ __launch_bounds__(256) void trmv_t_kernel(const TS* __restrict__ X, i
   const int64_t c = blockIdx.y;
   const int64_t nc = gridDim.y;
   const int64_t col0 = (int64_t)blockIdx.x * TRMV_TC;
-  const int64_t i0 = c * TRMV_RC;
-  const int64_t i1 = (i0 + TRMV_RC < np) ? i0 + TRMV_RC : np;
+  const int64_t i0 = c * rc;
+  const int64_t i1 = (i0 + rc < np) ? i0 + rc : np;
   if (i1 <= col0) return;
   __shared__ double rs[NV][TRMV_RC];
   __shared__ double red[NV][4][TRMV_TC];
-  for (int e = threadIdx.x; e < TRMV_RC; e += 256)
+  for (int e = threadIdx.x; e < rc; e += 256)
 #pragma unroll
     for (int q = 0; q < NV; ++q) rs[q][e] = (i0 + e < np) ? r[q * np + i0 + e] : 0.0;
   __syncthreads();
@@ -145,8 +149,9 @@ __global__ __launch_bounds__(256) void trmv_t_kernel(const TS* __restrict__ X, i
   }
 }
 
+// y (add: +=) the chunks' sums.
 __global__ void trmv_t_reduce(const double* __restrict__ partial, int64_t np, int64_t nchunks,
-                              int nv, double* __restrict__ y, Batch bt) {
+                              int64_t rc, int nv, int add, double* __restrict__ y, Batch bt) {
   if (bskip(bt)) return;
   partial = bws(partial, bt);
   y = bws(y, bt);
@@ -154,8 +159,8 @@ __global__ void trmv_t_reduce(const double* __restrict__ partial, int64_t np, in
   if (k >= np) return;
   for (int q = 0; q < nv; ++q) {
     double s = 0.0;
-    for (int64_t c = k / TRMV_RC; c < nchunks; ++c) s += partial[(q * nchunks + c) * np + k];
-    y[q * np + k] = s;
+    for (int64_t c = k / rc; c < nchunks; ++c) s += partial[(q * nchunks + c) * np + k];
+    y[q * np + k] = add ? y[q * np + k] + s : s;
   }
 }
 
@@ -241,8 +246,10 @@ __global__ __launch_bounds__(256) void sigma_mv_kernel(int kind, const double* _
   }
 }
 
+// y = the chunks' sums; res (optional) = r - y for the first vector.
 __global__ void sum_chunks(const double* __restrict__ partial, int64_t np, int64_t nchunks,
-                           int nv, double* __restrict__ y, Batch bt) {
+                           int nv, double* __restrict__ y, const double* __restrict__ r,
+                           double* __restrict__ res, Batch bt) {
   if (bskip(bt)) return;
   partial = bws(partial, bt);
   y = bws(y, bt);
@@ -250,8 +257,10 @@ __global__ void sum_chunks(const double* __restrict__ partial, int64_t np, int64
   if (i >= np) return;
   for (int q = 0; q < nv; ++q) {
     double s = 0.0;
+#pragma unroll 4
     for (int64_t c = 0; c < nchunks; ++c) s += partial[(q * nchunks + c) * np + i];
     y[q * np + i] = s;
+    if (q == 0 && res) bws(res, bt)[i] = bws(r, bt)[i] - s;
   }
 }
 
@@ -347,7 +356,9 @@ __global__ __launch_bounds__(256) void packed_symv_tile_kernel(const double* __r
 __global__ __launch_bounds__(512) void packed_symv_reduce(const double* __restrict__ prow,
                                                           const double* __restrict__ pcol,
                                                           int64_t T, int64_t ntile, int nv,
-                                                          double* __restrict__ v, Batch bt) {
+                                                          double* __restrict__ v,
+                                                          const double* __restrict__ r,
+                                                          double* __restrict__ res, Batch bt) {
   if (bskip(bt)) return;
   prow = bws(prow, bt);
   pcol = bws(pcol, bt);
@@ -366,38 +377,52 @@ __global__ __launch_bounds__(512) void packed_symv_reduce(const double* __restri
     }
     red[g][i] = acc;
     __syncthreads();
-    if (g == 0) v[q * np + I * NB + i] = ((red[0][i] + red[1][i]) + red[2][i]) + red[3][i];
+    if (g == 0) {
+      const double sum = ((red[0][i] + red[1][i]) + red[2][i]) + red[3][i];
+      v[q * np + I * NB + i] = sum;
+      if (q == 0 && res) bws(res, bt)[I * NB + i] = bws(r, bt)[I * NB + i] - sum;
+    }
     __syncthreads();
   }
 }
 
-// y_j partial over rows [c*RC, (c+1)*RC) of a dense rows x cols matrix:
+// y_j partial over rows [c*rc, (c+1)*rc) of a dense rows x cols matrix:
 // sum_i M[i][j] v_i, or sum_i M[i][j]^2 when v is null (rows i >= j only when
 // lower), float64 sums.  A block takes 64 columns; its four waves take every
-// fourth row of the chunk (wave w: rows c*RC + w, + 4, ...), each lane one
-// column, and their four sums are added in wave order.  With one thread per
-// column and 256 columns per block, the predictive's 16,384 x 4,096 passes ran
-// 256 blocks of one serial 1,024-row chain each, at about 1.1 TB/s.
+// fourth row of the chunk (wave w: rows c*rc + w, + 4, ...), each lane one
+// column, four rows in flight, and their sums are added in a fixed order.  With one
+// thread per column and 256 columns per block, the predictive's 16,384 x 4,096 passes
+// ran 256 blocks of one serial 1,024-row chain each, at about 1.1 TB/s.  Measured
+// (1,024-row chunks, one row in flight -> now): 2,048 x 512 100 -> 13 us,
+// 8,192 x 8,192 177 -> 121 us.
 template <typename TM>
 __global__ __launch_bounds__(256) void colreduce_kernel(const TM* __restrict__ M, int64_t ld,
-                                                        int64_t rows, int64_t cols,
+                                                        int64_t rows, int64_t cols, int64_t rc,
                                                         const double* __restrict__ v, int lower,
                                                         double* __restrict__ partial) {
   __shared__ double red[4][64];
   const int64_t c = blockIdx.y;
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int64_t j = (int64_t)blockIdx.x * 64 + lane;
-  const int64_t i0 = c * TRMV_RC;
-  const int64_t i1 = (i0 + TRMV_RC < rows) ? i0 + TRMV_RC : rows;
-  double acc = 0.0;
+  const int64_t j0 = (int64_t)blockIdx.x * 64;
+  const int64_t j = j0 + lane;
+  const int64_t i1 = ((c + 1) * rc < rows) ? (c + 1) * rc : rows;
+  int64_t i = c * rc + w;
+  // rows above the block's columns hold nothing of a lower triangle; the 64 rows of
+  // its diagonal are masked
+  if (lower && i < j0) i += (j0 - i + 3) / 4 * 4;
+  double a[4] = {0.0, 0.0, 0.0, 0.0};
   if (j < cols) {
-    for (int64_t i = i0 + w; i < i1; i += 4) {
-      if (lower && i < j) continue;
-      const double m = (double)M[i * ld + j];
-      acc += v ? m * v[i] : m * m;
+    auto term = [&](int64_t r) {
+      const double m = (lower && r < j) ? 0.0 : (double)M[r * ld + j];
+      return v ? m * v[r] : m * m;
+    };
+    for (; i + 12 < i1; i += 16) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) a[u] += term(i + 4 * u);
     }
+    for (; i < i1; i += 4) a[0] += term(i);
   }
-  red[w][lane] = acc;
+  red[w][lane] = (a[0] + a[1]) + (a[2] + a[3]);
   __syncthreads();
   if (w == 0 && j < cols)
     partial[c * cols + j] = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
@@ -408,6 +433,7 @@ __global__ void colreduce_sum(const double* __restrict__ partial, int64_t cols, 
   const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= cols) return;
   double s = 0.0;
+#pragma unroll 4
   for (int64_t c = 0; c < nchunks; ++c) s += partial[c * cols + j];
   y[j] = s;
 }
@@ -440,7 +466,7 @@ __global__ void mfma_selftest_kernel(double* out64, float* outbf) {
 
 template <typename TS>
 int launch_trmv(const TS* X, int64_t ld, int64_t np, const double* r, double* y, bool trans,
-                double* partial, hipStream_t s, const Batch& bt, int nv) {
+                double* partial, hipStream_t s, const Batch& bt, int nv, bool add) {
   if (np % NB) {
     set_error("trmv: size %lld not a multiple of %d", (long long)np, NB);
     return GPK_ERR_BAD_ARG;
@@ -452,35 +478,47 @@ int launch_trmv(const TS* X, int64_t ld, int64_t np, const double* r, double* y,
   const dim3 gvec((unsigned)((np + 255) / 256), 1, bt.count);
   if (!trans) {
     const int64_t nc = (np + TRMV_CW - 1) / TRMV_CW;
-    const dim3 grid((unsigned)(np / 16), (unsigned)nc, bt.count);
-    if (nv == 1)
-      hipLaunchKernelGGL((trmv_n_kernel<TS, 1>), grid, dim3(256), 0, s, X, ld, np, r, partial, bt);
-    else
-      hipLaunchKernelGGL((trmv_n_kernel<TS, 3>), grid, dim3(256), 0, s, X, ld, np, r, partial, bt);
+    // one chunk: the rows' sums are the result
+    double* out = nc == 1 ? y : partial;
+    const bool narrow = np / 16 * nc * bt.count < 1024;
+    const dim3 grid((unsigned)(np / (narrow ? 4 : 16)), (unsigned)nc, bt.count);
+#define GPK_TRMV_N(NV, RW) \
+  hipLaunchKernelGGL((trmv_n_kernel<TS, NV, RW>), grid, dim3(256), 0, s, X, ld, np, r, out, bt)
+    if (nv == 1 && narrow) GPK_TRMV_N(1, 1);
+    else if (nv == 1) GPK_TRMV_N(1, 4);
+    else if (narrow) GPK_TRMV_N(3, 1);
+    else GPK_TRMV_N(3, 4);
+#undef GPK_TRMV_N
     GPK_LAUNCH_CHECK();
-    hipLaunchKernelGGL(trmv_n_reduce, gvec, dim3(256), 0, s, partial, np, nc, nv, y, bt);
+    if (nc > 1)
+      hipLaunchKernelGGL(trmv_n_reduce, gvec, dim3(256), 0, s, partial, np, nc, nv, y, bt);
   } else {
-    const int64_t nc = (np + TRMV_RC - 1) / TRMV_RC;
+    const int64_t rc = trmv_t_rows(np, bt.count);
+    const int64_t nc = (np + rc - 1) / rc;
     const dim3 grid((unsigned)(np / TRMV_TC), (unsigned)nc, bt.count);
     if (nv == 1)
-      hipLaunchKernelGGL((trmv_t_kernel<TS, 1>), grid, dim3(256), 0, s, X, ld, np, r, partial, bt);
+      hipLaunchKernelGGL((trmv_t_kernel<TS, 1>), grid, dim3(256), 0, s, X, ld, np, rc, r, partial,
+                         bt);
     else
-      hipLaunchKernelGGL((trmv_t_kernel<TS, 3>), grid, dim3(256), 0, s, X, ld, np, r, partial, bt);
+      hipLaunchKernelGGL((trmv_t_kernel<TS, 3>), grid, dim3(256), 0, s, X, ld, np, rc, r, partial,
+                         bt);
     GPK_LAUNCH_CHECK();
-    hipLaunchKernelGGL(trmv_t_reduce, gvec, dim3(256), 0, s, partial, np, nc, nv, y, bt);
+    hipLaunchKernelGGL(trmv_t_reduce, gvec, dim3(256), 0, s, partial, np, nc, rc, nv, add ? 1 : 0,
+                       y, bt);
   }
   GPK_LAUNCH_CHECK();
   return GPK_OK;
 }
 
 template int launch_trmv<double>(const double*, int64_t, int64_t, const double*, double*, bool,
-                                 double*, hipStream_t, const Batch&, int);
+                                 double*, hipStream_t, const Batch&, int, bool);
 template int launch_trmv<float>(const float*, int64_t, int64_t, const double*, double*, bool,
-                                double*, hipStream_t, const Batch&, int);
+                                double*, hipStream_t, const Batch&, int, bool);
 
 int launch_sigma_matvec(int kind, const double* x, int64_t n, int64_t np, int d,
                         const double* theta, int nls, double jitter, const double* a, double* v,
-                        double* partial, hipStream_t s, const Batch& bt, int nv) {
+                        double* partial, hipStream_t s, const Batch& bt, int nv, const double* r,
+                        double* res) {
   if (d < 1 || d > MAX_D) {
     set_error("sigma matvec: input dimension %d outside [1, %d]", d, MAX_D);
     return GPK_ERR_BAD_ARG;
@@ -511,13 +549,14 @@ int launch_sigma_matvec(int kind, const double* x, int64_t n, int64_t np, int d,
 #undef GPK_SMV
   GPK_LAUNCH_CHECK();
   hipLaunchKernelGGL(sum_chunks, dim3((unsigned)((np + 255) / 256), 1, bt.count), dim3(256), 0, s,
-                     partial, np, nc, nv, v, bt);
+                     partial, np, nc, nv, v, r, res, bt);
   GPK_LAUNCH_CHECK();
   return GPK_OK;
 }
 
 int launch_packed_symv(const double* S, int64_t np, const double* a, double* v,
-                       double* partial, hipStream_t s, const Batch& bt, int nv) {
+                       double* partial, hipStream_t s, const Batch& bt, int nv, const double* r,
+                       double* res) {
   if (np % NB) {
     set_error("packed symv: size %lld not a multiple of %d", (long long)np, NB);
     return GPK_ERR_BAD_ARG;
@@ -542,7 +581,7 @@ int launch_packed_symv(const double* S, int64_t np, const double* a, double* v,
                        ntile, bt);
   GPK_LAUNCH_CHECK();
   hipLaunchKernelGGL(packed_symv_reduce, dim3((unsigned)T, 1, bt.count), dim3(512), 0, s, prow,
-                     pcol, T, ntile, nv, v, bt);
+                     pcol, T, ntile, nv, v, r, res, bt);
   GPK_LAUNCH_CHECK();
   return GPK_OK;
 }
@@ -551,9 +590,10 @@ template <typename TM>
 int launch_colreduce(const TM* M, int64_t ld, int64_t rows, int64_t cols, const double* v,
                      double* y, double* partial, hipStream_t s, bool lower) {
   if (rows <= 0 || cols <= 0) return GPK_OK;
-  const int64_t nc = (rows + TRMV_RC - 1) / TRMV_RC;
+  const int64_t rc = colreduce_rows(rows);
+  const int64_t nc = (rows + rc - 1) / rc;
   hipLaunchKernelGGL(colreduce_kernel<TM>, dim3((unsigned)((cols + 63) / 64), (unsigned)nc),
-                     dim3(256), 0, s, M, ld, rows, cols, v, lower ? 1 : 0, partial);
+                     dim3(256), 0, s, M, ld, rows, cols, rc, v, lower ? 1 : 0, partial);
   GPK_LAUNCH_CHECK();
   hipLaunchKernelGGL(colreduce_sum, dim3((unsigned)((cols + 255) / 256)), dim3(256), 0, s,
                      partial, cols, nc, y);
