@@ -306,6 +306,140 @@ __global__ __launch_bounds__(WaveLayout<AR>::NT) void adjoint_kernel(int kind,
   }
 }
 
+// The FP64 pass on 64 x 64 tiles (inputs of up to ADJ_DCH dimensions), for problems
+// whose 128-tiles leave most of the chip idle: four independent waves of 32 x 32, each
+// reading its operands straight from global memory (DirectLoop).  Tiles (I, J),
+// I >= J, of 64 rows; each writes its own partial sums.  k runs from the row tile at
+// the granularity of KG, in the large tiles' order.  np = 2,048: 285 us on 136 large
+// tiles, 158 us.
+constexpr int AT = 64;
+template <int DMAX, bool XT>
+__global__ __launch_bounds__(256, 2) void adjoint_small_kernel(
+    int kind, const double* __restrict__ X, int64_t ld, int64_t np, const double* __restrict__ x,
+    int64_t n, int d, const double* __restrict__ theta, int nls, const double* __restrict__ alpha,
+    const double* __restrict__ beta, int dense, double* __restrict__ partial, Batch bt) {
+  __shared__ double xm[AT][DMAX + 1], xn[AT][DMAX + 1];
+  __shared__ double am[AT], an[AT], bm[AT], bn[AT];
+  __shared__ double red_s[4][DMAX + 2];
+  bmember(bt, d, x, n, theta);
+  X = bws(X, bt);
+  alpha = bws(alpha, bt);
+  beta = bws(beta, bt);
+  partial = bws(partial, bt);
+  int64_t mt, nt;
+  lower_tile(blockIdx.x, mt, nt);
+  const int64_t m0 = mt * AT, n0 = nt * AT;
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int64_t mw = m0 + (w >> 1) * 32, nw = n0 + (w & 1) * 32;
+  f64x4 acc[2][2];
+  DirectLoop<!XT, !XT, 2, 2> loop(X, ld, X, ld, mw, nw, lane, dense ? 0 : m0 / KG * KG, np);
+  for (int e = t; e < AT * DMAX; e += 256) {
+    const int r = e / DMAX, q = e % DMAX;
+    if (q < d) {
+      const double l = theta[nls == 1 ? 0 : q];
+      xm[r][q] = m0 + r < n ? x[(m0 + r) * d + q] / l : 0.0;
+      xn[r][q] = n0 + r < n ? x[(n0 + r) * d + q] / l : 0.0;
+    }
+  }
+  if (t < AT) {
+    am[t] = alpha[m0 + t];
+    an[t] = alpha[n0 + t];
+    if (beta) {
+      bm[t] = beta[m0 + t];
+      bn[t] = beta[n0 + t];
+    }
+  }
+  loop.run(acc);
+  __syncthreads();
+
+  const double wt = (mt == nt) ? 1.0 : 2.0;
+  const bool ard = nls > 1;
+  const int nv = nls + 2;
+  const int lr = lane >> 4, lc = lane & 15;
+  double s_var = 0.0, s_tr = 0.0, s_ls[DMAX];
+#pragma unroll
+  for (int q = 0; q < DMAX; ++q) s_ls[q] = 0.0;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int lj = (w & 1) * 32 + 16 * j + lc;
+      const int64_t gj = n0 + lj;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int li = (w >> 1) * 32 + 16 * i + lr + 4 * r;
+        const int64_t gi = m0 + li;
+        if (gi >= n || gj >= n) continue;
+        const double wij =
+            (beta ? am[li] * bn[lj] + bm[li] * an[lj] : am[li] * an[lj]) - acc[i][j][r];
+        double d2 = 0.0;
+#pragma unroll
+        for (int q = 0; q < DMAX; ++q) {
+          if (q < d) {
+            const double df = xm[li][q] - xn[lj][q];
+            d2 += df * df;
+          }
+        }
+        double kv, fv;
+        kval_fac(kind, d2, kv, fv);
+        const double g = wt * wij;
+        s_var += g * kv;
+        if (gi == gj) s_tr += wij;
+        const double gf = g * fv;
+        if (ard) {
+#pragma unroll
+          for (int q = 0; q < DMAX; ++q) {
+            if (q < d) {
+              const double df = xm[li][q] - xn[lj][q];
+              s_ls[q] += gf * df * df;
+            }
+          }
+        } else {
+          s_ls[0] += gf * d2;
+        }
+      }
+    }
+#pragma unroll
+  for (int q = 0; q < DMAX + 2; ++q) {
+    double v = q < DMAX ? s_ls[q] : (q == DMAX ? s_var : s_tr);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+    if (lane == 0) red_s[w][q] = v;
+  }
+  __syncthreads();
+  if (t < nv) {
+    const int q = t < nls ? t : (t == nls ? DMAX : DMAX + 1);
+    partial[(int64_t)blockIdx.x * nv + t] =
+        ((red_s[0][q] + red_s[1][q]) + red_s[2][q]) + red_s[3][q];
+  }
+}
+
+int launch_small_adjoint(int kind, const double* X, int64_t ld, int64_t np, const double* x,
+                         int64_t n, int d, const double* theta, int nls, const double* alpha,
+                         double* partial, hipStream_t s, const Batch& bt, const double* beta,
+                         bool dense, bool xt) {
+  const int64_t nt = np / AT;
+  const dim3 grid((unsigned)(nt * (nt + 1) / 2), 1, bt.count);
+#define GPK_ADJS(DM)                                                                          \
+  do {                                                                                        \
+    if (xt)                                                                                   \
+      hipLaunchKernelGGL((adjoint_small_kernel<DM, true>), grid, dim3(256), 0, s, kind, X, ld, \
+                         np, x, n, d, theta, nls, alpha, beta, dense ? 1 : 0, partial, bt);   \
+    else                                                                                      \
+      hipLaunchKernelGGL((adjoint_small_kernel<DM, false>), grid, dim3(256), 0, s, kind, X,   \
+                         ld, np, x, n, d, theta, nls, alpha, beta, dense ? 1 : 0, partial, bt); \
+  } while (0)
+  if (d <= 1) GPK_ADJS(1);
+  else if (d <= 2) GPK_ADJS(2);
+  else if (d <= 4) GPK_ADJS(4);
+  else if (d <= 8) GPK_ADJS(8);
+  else if (d <= 16) GPK_ADJS(16);
+  else GPK_ADJS(32);
+#undef GPK_ADJS
+  GPK_LAUNCH_CHECK();
+  return GPK_OK;
+}
+
 template <int AR, typename TS>
 int launch_ar(int kind, const TS* X, int64_t ld, int64_t np, const double* x, int64_t n, int d,
               const double* theta, int nls, const double* alpha, double* partial,
@@ -350,6 +484,11 @@ int launch_adjoint(int kind, int arith, const TS* X, int64_t ld, int64_t np, con
   if (np % TILE) {
     set_error("adjoint: padded size %lld not a multiple of %d", (long long)np, TILE);
     return GPK_ERR_BAD_ARG;
+  }
+  if constexpr (std::is_same<TS, double>::value) {
+    if (arith == AR_F64 && adjoint_small(np, d, bt.count))
+      return launch_small_adjoint(kind, X, ld, np, x, n, d, theta, nls, alpha, partial, s, bt,
+                                  beta, dense, xt);
   }
   if (arith == AR_F64)
     return launch_ar<AR_F64, TS>(kind, X, ld, np, x, n, d, theta, nls, alpha, partial, s, bt,

@@ -168,7 +168,8 @@ Layout make_layout(int64_t n, int64_t d, int prec, int spk = -1) {
   o += al(L.has_spk ? (size_t)2 * L.nvec * ntile * NB * sizeof(double) : 0);
   L.off_part = o; o += al((size_t)L.nvec * nchunk * np * sizeof(double));
   L.off_skip = o; o += al(sizeof(int));
-  L.off_gpart = o; o += al((size_t)ntile * (d + 2) * sizeof(double));
+  L.off_gpart = o;
+  o += al((size_t)adjoint_tiles(prec == GPK_PREC_FP64, np, (int)d, 1) * (d + 2) * sizeof(double));
   L.off_scal = o; o += al(16 * sizeof(double));
   L.off_probe = o; o += al(3 * NPROBE * sizeof(double));
   L.total = o;
@@ -648,9 +649,8 @@ int mll_backward_t(int kind, const Arith3& ar, const double* x, int64_t n, int d
                                np, x, n, d, theta, nls, at<double>(ws, Lo.off_alpha), gpart, s,
                                bt, nullptr, false, fs));
   }
-  const int64_t nleaf = np / NB;
   hipLaunchKernelGGL(finalize_bwd_kernel, dim3((unsigned)(nls + 3), 1, bt.count), dim3(256), 0, s,
-                     gpart, nleaf * (nleaf + 1) / 2, nls, theta, at<double>(ws, Lo.off_alpha), n,
+                     gpart, adjoint_tiles(f64, np, d, bt.count), nls, theta, at<double>(ws, Lo.off_alpha), n,
                      gbar, grad, bt);
   GPK_LAUNCH_CHECK();
   return GPK_OK;
@@ -922,9 +922,8 @@ int loocv_backward_t(int kind, const Arith3& ar3, const double* x, int64_t n, in
   double* gpart = at<double>(ws, Lo.off_gpart);
   GPK_TRY(launch_adjoint<TS>(kind, ar, Y, np, np, x, n, d, theta, nls,
                              at<double>(ws, Lo.off_alpha), gpart, s, Batch(), w, true));
-  const int64_t nleaf = np / NB;
   hipLaunchKernelGGL(finalize_bwd_kernel, dim3((unsigned)(nls + 3)), dim3(256), 0, s, gpart,
-                     nleaf * (nleaf + 1) / 2, nls, theta, w, n, gbar, grad, Batch());
+                     adjoint_tiles(f64, np, d, 1), nls, theta, w, n, gbar, grad, Batch());
   GPK_LAUNCH_CHECK();
   return GPK_OK;
 }

@@ -164,22 +164,6 @@ __global__ __launch_bounds__(WaveLayout<AR>::NT) void gemm_kernel(GemmParams p) 
 // of 64 cycles per slab and wave.  Measured per launch: K = 128, one to sixteen
 // 128-tiles 24 -> 6 us; the 1,024 x 1,024 x 1,024 products of the triangular
 // inverse 142 -> 51 us.
-constexpr int SETS = 4;
-constexpr int SLAB = 16;
-
-template <bool KM>
-__device__ __forceinline__ void frag_load(const double* __restrict__ P, int64_t ld, int64_t row,
-                                          int64_t k, double (&v)[4]) {
-  if (!KM) {
-    const double2* q = reinterpret_cast<const double2*>(P + row * ld + k);
-    const double2 a = q[0], b = q[1];
-    v[0] = a.x; v[1] = a.y; v[2] = b.x; v[3] = b.y;
-  } else {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) v[q] = P[(k + q) * ld + row];
-  }
-}
-
 template <bool A_KM, bool B_KN, int MI, int NJ>
 __global__ __launch_bounds__(256, 2) void gemm_small_kernel(GemmParams p) {
   constexpr int BM = 32 * MI, BN = 32 * NJ;
@@ -189,7 +173,6 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(GemmParams p) {
   if (!gemm_tile(p, blockIdx.x / (SM * SN), mt, nt)) return;
   const int sub = blockIdx.x % (SM * SN);
   const int64_t m0 = mt * TILE + (sub / SN) * BM, n0 = nt * TILE + (sub % SN) * BN;
-  constexpr int64_t KG = SETS * SLAB;
   int64_t kb = 0, ke = p.K;
   if (p.krange == KR_GE_N) kb = n0 / KG * KG;
   else if (p.krange == KR_LE_M) ke = min(p.K, (m0 + BM + KG - 1) / KG * KG);
@@ -201,22 +184,8 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(GemmParams p) {
   const double* A = static_cast<const double*>(p.A);
   const double* B = static_cast<const double*>(p.B);
   double* C = static_cast<double*>(p.C);
-  double av[SETS][MI][4], bv[SETS][NJ][4];
-  auto load = [&](int s, int64_t k) {
-#pragma unroll
-    for (int i = 0; i < MI; ++i) frag_load<A_KM>(A, p.lda, mw + 16 * i + lc, k + 4 * lr, av[s][i]);
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) frag_load<B_KN>(B, p.ldb, nw + 16 * j + lc, k + 4 * lr, bv[s][j]);
-  };
   f64x4 acc[MI][NJ];
-#pragma unroll
-  for (int i = 0; i < MI; ++i)
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
-  if (kb < ke) {
-#pragma unroll
-    for (int s = 0; s < SETS; ++s) load(s, kb + s * SLAB);
-  }
+  DirectLoop<A_KM, B_KN, MI, NJ> loop(A, p.lda, B, p.ldb, mw, nw, lane, kb, ke);
   double cv[MI][NJ][4];
 #pragma unroll
   for (int i = 0; i < MI; ++i)
@@ -226,20 +195,7 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(GemmParams p) {
       for (int r = 0; r < 4; ++r)
         cv[i][j][r] =
             p.beta_one ? C[(mw + 16 * i + lr + 4 * r) * p.ldc + nw + 16 * j + lc] : 0.0;
-  for (int64_t k = kb; k < ke; k += KG) {
-#pragma unroll
-    for (int s = 0; s < SETS; ++s) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-          for (int j = 0; j < NJ; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[s][i][q], bv[s][j][q], acc[i][j],
-                                                             0, 0, 0);
-      if (k + KG < ke) load(s, k + KG + s * SLAB);
-    }
-  }
+  loop.run(acc);
 #pragma unroll
   for (int i = 0; i < MI; ++i)
 #pragma unroll

@@ -179,6 +179,75 @@ __device__ __forceinline__ void mfma_slab_f64(const double* a, const double* b, 
 }
 
 // ---------------------------------------------------------------------------
+// float64 main loop of the small tiles: operands straight from global memory
+// ---------------------------------------------------------------------------
+constexpr int SETS = 4;
+constexpr int SLAB = 16;
+
+template <bool KM>
+__device__ __forceinline__ void frag_load(const double* __restrict__ P, int64_t ld, int64_t row,
+                                          int64_t k, double (&v)[4]) {
+  if (!KM) {
+    const double2* q = reinterpret_cast<const double2*>(P + row * ld + k);
+    const double2 a = q[0], b = q[1];
+    v[0] = a.x; v[1] = a.y; v[2] = b.x; v[3] = b.y;
+  } else {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = P[(k + q) * ld + row];
+  }
+}
+
+// acc(m, n) = sum over k in [kb, ke) of one wave's 16 MI x 16 NJ tile at (mw, nw),
+// kb and ke multiples of KG (or kb >= ke).  Constructed before the loads that
+// should overlap its first slabs' latency, run afterwards.
+constexpr int64_t KG = SETS * SLAB;
+template <bool A_KM, bool B_KN, int MI, int NJ>
+struct DirectLoop {
+  const double* A;
+  int64_t lda;
+  const double* B;
+  int64_t ldb;
+  int64_t mw, nw, kb, ke;
+  int lr, lc;
+  double av[SETS][MI][4], bv[SETS][NJ][4];
+  __device__ __forceinline__ void load(int s, int64_t k) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i) frag_load<A_KM>(A, lda, mw + 16 * i + lc, k + 4 * lr, av[s][i]);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) frag_load<B_KN>(B, ldb, nw + 16 * j + lc, k + 4 * lr, bv[s][j]);
+  }
+  __device__ __forceinline__ DirectLoop(const double* a, int64_t la, const double* b, int64_t lb,
+                                        int64_t m, int64_t n, int lane, int64_t k0, int64_t k1)
+      : A(a), lda(la), B(b), ldb(lb), mw(m), nw(n), kb(k0), ke(k1), lr(lane >> 4),
+        lc(lane & 15) {
+    if (kb < ke) {
+#pragma unroll
+      for (int s = 0; s < SETS; ++s) load(s, kb + s * SLAB);
+    }
+  }
+  __device__ __forceinline__ void run(f64x4 (&acc)[MI][NJ]) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
+    for (int64_t k = kb; k < ke; k += KG) {
+#pragma unroll
+      for (int s = 0; s < SETS; ++s) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[s][i][q], bv[s][j][q],
+                                                               acc[i][j], 0, 0, 0);
+        if (k + KG < ke) load(s, k + KG + s * SLAB);
+      }
+    }
+  }
+};
+
+// ---------------------------------------------------------------------------
 // float64 main loop
 // ---------------------------------------------------------------------------
 template <typename TA, typename TB, bool A_KM, bool B_KN>

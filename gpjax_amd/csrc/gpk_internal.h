@@ -310,10 +310,25 @@ int launch_tri_level(int arith, const TriLevel& lev, int64_t max_m, int64_t max_
 int launch_trsm_strip(double* B, int64_t ld, int64_t m, const double* inv, hipStream_t s,
                       const Batch& bt = Batch());
 
+// True when the FP64 pass below runs on 64-tiles, and the number of partial records a
+// call writes (each nls + 2 doubles): one per tile.  Up to 600 128-tiles, about
+// where those fill the chip's two workgroups per CU: MLL + gradient at n = 2,000 1.60
+// -> 1.47 ms and n = 4,000 even, but n = 6,000 (1,128 tiles) 8.5 -> 8.9 ms and a batch
+// of 4,096 small GPs 60.8 -> 62.6 ms with the small tiles.
+constexpr int64_t ADJ_SMALL_TILES = 600;
+inline bool adjoint_small(int64_t np, int d, int64_t members) {
+  const int64_t T = np / NB;
+  return d <= 32 && T * (T + 1) / 2 * members <= ADJ_SMALL_TILES;
+}
+inline int64_t adjoint_tiles(bool f64, int64_t np, int d, int64_t members) {
+  const int64_t T = f64 && adjoint_small(np, d, members) ? np / 64 : np / NB;
+  return T * (T + 1) / 2;
+}
+
 // Fused LAUUM + adjoint: for every lower NB-tile of Sinv = X^T X (X = L^-1,
 // lower, Np x Np), reduce 1/2 tr(W dSigma/dtheta) contributions with
 // W = alpha alpha^T - Sinv against kernel tiles recomputed from x.
-// partial: [num_tiles][nls + 2] float64.
+// partial: [adjoint_tiles][nls + 2] float64.
 // beta (optional): W = alpha beta^T + beta alpha^T - X^T X instead; dense: X is
 // a dense Np x Np matrix (every k) rather than lower triangular (k >= row).
 // fscale (AR_FP16X3 only): device pointer to the power-of-two scale of X.
