@@ -488,12 +488,20 @@ int check_ws(const char* fn, const void* ws, size_t have, size_t need) {
 //   evaluating the kernel again;
 // adj_transposed: the fused Sigma^-1 pass reads U = X^T along k (one transpose
 //   first) instead of X down its columns.
-// The single-problem path runs the defaults; the batched path takes them per
-// size group from the autotuner's table.
+// The single-problem path runs the defaults (single_variant); the batched path takes
+// them per size group from the autotuner's table.
 struct Variant {
   bool stored_sigma = true;
   bool adj_transposed = true;
 };
+// A single problem's: the FP64 pass on small tiles reads its operands straight into
+// the matrix cores, where a column read takes whole 128-byte lines and a row read
+// touches 16 lines per instruction (n = 2,000: 158 -> 115 us and no transpose).
+Variant single_variant(bool f64, int64_t np, int d) {
+  Variant v;
+  v.adj_transposed = !(f64 && adjoint_small(np, d, 1));
+  return v;
+}
 
 template <typename TS>
 int mll_forward_t(int kind, const Arith3& ar, const double* x, const double* y, int64_t n, int d,
@@ -628,9 +636,10 @@ template <typename TS>
 int mll_backward_t(int kind, const Arith3& ar, const double* x, int64_t n, int d,
                    const double* theta, int nls, double gbar, void* ws, const Layout& Lo,
                    double* grad, hipStream_t s, const Batch& bt = Batch(),
-                   const Variant& vr = Variant()) {
+                   const Variant* variant = nullptr) {
   const int64_t np = Lo.np;
   const bool f64 = std::is_same<TS, double>::value;
+  const Variant vr = variant ? *variant : single_variant(f64, np, d);
   double* gpart = at<double>(ws, Lo.off_gpart);
   const float* fs = f64 ? nullptr : at<float>(ws, Lo.off_scal) + 2;
   if (vr.adj_transposed) {
@@ -786,7 +795,7 @@ int predict_t(int kind, const Arith3& ar, const double* x, const double* y, int6
 // w = Sigma^-1 v, c_i^2 = 1/d_i + alpha_i^2/d_i^2 and
 //   W = alpha w^T + w alpha^T - Y^T Y,   Y = diag(c) Sigma^-1,
 // which the adjoint pass reduces against dSigma/dtheta with Y dense.
-// Sigma^-1 = X^T X is formed (lower tiles, mirrored and row-scaled in place)
+// Sigma^-1 = X^T X is formed (lower tiles, mirrored and scaled in place)
 // in the buffer that held L, which the backward no longer needs.
 struct LooLayout {
   size_t off_d = 0, off_v = 0, off_w = 0, off_c = 0, off_tmp = 0, off_mres = 0, total = 0;
@@ -842,9 +851,12 @@ __global__ __launch_bounds__(256) void loo_fwd_kernel(const double* __restrict__
   }
 }
 
-// Y <- diag(c) S with S symmetric held in its lower 64-tiles (upper tiles are
-// overwritten).  One workgroup per lower tile (I, J): it reads only tile (I, J)
-// and writes tiles (I, J) and (J, I), so the update in place has no race.
+// Y <- diag(c) S, or its transpose S diag(c) (tr), with S symmetric held in its lower
+// 64-tiles (upper tiles are overwritten).  The transpose lets the pass over Y^T Y
+// read both operands along rows (n = 9,000 float64 34.7 -> 33.5 ms, n = 16,000 mixed
+// 63.2 -> 62.4); its small tiles prefer columns (single_variant).  One workgroup per
+// lower tile (I, J): it reads only tile (I, J) and writes tiles (I, J) and (J, I), so
+// the update in place has no race.
 constexpr int MT = 64;
 // Lower-triangle tile t -> (I, J), I >= J, row-major over I.
 __device__ __forceinline__ void tri_tile(int64_t t, int64_t& I, int64_t& J) {
@@ -857,7 +869,8 @@ __device__ __forceinline__ void tri_tile(int64_t t, int64_t& I, int64_t& J) {
 
 template <typename TS>
 __global__ __launch_bounds__(256) void loo_scale_mirror_kernel(TS* __restrict__ Y, int64_t ld,
-                                                               const double* __restrict__ c) {
+                                                               const double* __restrict__ c,
+                                                               int tr) {
   __shared__ TS tl[MT][MT + 1];
   int64_t I, J;
   tri_tile(blockIdx.x, I, J);
@@ -869,12 +882,15 @@ __global__ __launch_bounds__(256) void loo_scale_mirror_kernel(TS* __restrict__ 
   __syncthreads();
   for (int e = threadIdx.x; e < MT * MT; e += 256) {
     const int r = e / MT, q = e % MT;
+    // entry (r0 + r, c0 + q) and its mirror (c0 + r, r0 + q)
+    const double cl = tr ? c[c0 + q] : c[r0 + r];
     if (I == J) {
       const TS sv = r >= q ? tl[r][q] : tl[q][r];
-      Y[(r0 + r) * ld + c0 + q] = (TS)(c[r0 + r] * (double)sv);
+      Y[(r0 + r) * ld + c0 + q] = (TS)(cl * (double)sv);
     } else {
-      Y[(r0 + r) * ld + c0 + q] = (TS)(c[r0 + r] * (double)tl[r][q]);
-      Y[(c0 + r) * ld + r0 + q] = (TS)(c[c0 + r] * (double)tl[q][r]);
+      const double cu = tr ? c[r0 + q] : c[c0 + r];
+      Y[(r0 + r) * ld + c0 + q] = (TS)(cl * (double)tl[r][q]);
+      Y[(c0 + r) * ld + r0 + q] = (TS)(cu * (double)tl[q][r]);
     }
   }
 }
@@ -912,16 +928,18 @@ int loocv_backward_t(int kind, const Arith3& ar3, const double* x, int64_t n, in
   GPK_TRY(launch_trmv<TS>(X, np, np, at<double>(ws, P.off_v), at<double>(ws, P.off_tmp), false,
                           part, s));
   GPK_TRY(launch_trmv<TS>(X, np, np, at<double>(ws, P.off_tmp), w, true, part, s));
-  // Y = diag(c) X^T X
+  // Y = diag(c) X^T X (or its transpose)
   GPK_TRY(launch_gemm<TS, TS, TS>(ar, true, true, X, np, X, np, Y, np, np, np, np, 1.0, false,
                                   true, KR_GE_M, s));
   const int64_t mt = np / MT;
+  const Variant vr = single_variant(f64, np, d);
   hipLaunchKernelGGL(loo_scale_mirror_kernel<TS>, dim3((unsigned)(mt * (mt + 1) / 2)), dim3(256),
-                     0, s, Y, np, at<double>(ws, P.off_c));
+                     0, s, Y, np, at<double>(ws, P.off_c), vr.adj_transposed ? 1 : 0);
   GPK_LAUNCH_CHECK();
   double* gpart = at<double>(ws, Lo.off_gpart);
   GPK_TRY(launch_adjoint<TS>(kind, ar, Y, np, np, x, n, d, theta, nls,
-                             at<double>(ws, Lo.off_alpha), gpart, s, Batch(), w, true));
+                             at<double>(ws, Lo.off_alpha), gpart, s, Batch(), w, true, nullptr,
+                             vr.adj_transposed));
   hipLaunchKernelGGL(finalize_bwd_kernel, dim3((unsigned)(nls + 3)), dim3(256), 0, s, gpart,
                      adjoint_tiles(f64, np, d, 1), nls, theta, w, n, gbar, grad, Batch());
   GPK_LAUNCH_CHECK();
@@ -1116,7 +1134,7 @@ int run_group(int kind, const Arith3& ar, const double* x, const double* y, int 
   // n is taken per member inside the kernels; np fixes the shapes.
   GPK_TRY(mll_forward_t<TS>(kind, ar, x, y, g.np, d, theta, nls, jitter, iters, wsg, g.lo,
                             result, s, bt, vr));
-  return mll_backward_t<TS>(kind, ar, x, g.np, d, theta, nls, 1.0, wsg, g.lo, grad, s, bt, vr);
+  return mll_backward_t<TS>(kind, ar, x, g.np, d, theta, nls, 1.0, wsg, g.lo, grad, s, bt, &vr);
 }
 
 template <typename TS>
