@@ -573,11 +573,8 @@ int mll_forward_t(int kind, const Arith3& ar, const double* x, const double* y, 
   }
   {
     PhaseScope ps(GPK_PHASE_POTRF, s);
-    const int64_t la = bt.gp ? 0 : lookahead_width(np, std::is_same<TS, float>::value);
-    if (la > 0)
-      GPK_TRY(F.potrf_lookahead(np, la));
-    else
-      GPK_TRY(F.potrf(0, np));
+    if (bt.gp) GPK_TRY(F.potrf(0, np));
+    else GPK_TRY(F.factor(np, true));
   }
   {
     PhaseScope ps(GPK_PHASE_TRTRI, s);

@@ -29,8 +29,16 @@ constexpr int64_t TRSM_STRIP_TILES = 512;
 static_assert(TRSM_STRIP_TILES >= SMALL_TILES, "an in-place product on small tiles would race");
 constexpr unsigned TRI_NODEWISE = 64;  // members from which the inverse goes node by node
 
+// Largest single float64 problem factored leaf by leaf on one stream
+// (Factor::potrf_steps).  Beyond it the trailing updates, a rank-128 step each, take
+// longer than the leaf they run beside.  MLL + gradient (two streams with the
+// look-ahead / leaf by leaf, ms): n = 2,000 1.41 / 1.04, n = 3,001 (leave-one-out)
+// 3.16 / 2.67, n = 4,000 3.80 / 3.37, n = 6,000 8.5 / 8.7, n = 8,000 15.6 / 17.3.
+constexpr int64_t STEPS_MAX = 4096;
+
 // Panel width of the look-ahead Cholesky (Factor::potrf_lookahead) for a single
-// np x np problem, np >= 2,048: np/32 with float32 storage, np/64 in float64,
+// np x np problem, np >= 2,048 (float64: > STEPS_MAX): np/32 with float32 storage, np/64
+// in float64,
 // rounded down to a multiple of NB, at least NB.  Wider panels put more of the
 // update into large rank-B GEMMs; narrower ones shorten the second stream's
 // chain per panel, which the first and last panels wait for.  Measured (ms per
@@ -151,6 +159,34 @@ struct Factor {
                                     n - h, n - h, h, -1.0, true, true, KR_FULL, s,
                                     dblk_at(o + h), bt, fscale));
     return potrf(o + h, n - h);
+  }
+  // The whole factorisation of one problem (no batch).  `streams`: the look-ahead may
+  // use this thread's second stream.
+  int factor(int64_t n, bool streams) {
+    const bool f32 = std::is_same<TS, float>::value;
+    if (!f32 && n <= STEPS_MAX) return potrf_steps(n);
+    const int64_t la = streams ? lookahead_width(n, f32) : 0;
+    return la > 0 ? potrf_lookahead(n, la) : potrf(0, n);
+  }
+  // Right-looking in single leaves on one stream (float64): per leaf a launch of the
+  // leaf beside the trailing update by the panel before it, one of the column block's
+  // solve, and one of the next column block's update.
+  int potrf_steps(int64_t n) {
+    if constexpr (std::is_same<TS, double>::value) {
+      GPK_TRY(leaf(0));
+      for (int64_t o = 0; o + NB < n; o += NB) {
+        const int64_t o1 = o + NB, rest = n - o1 - NB;
+        GPK_TRY(trsm(o1, n - o1, o, NB));
+        const TS* P = L + o1 * ld + o;
+        GPK_TRY(launch_gemm<TS, TS, TS>(AR_F64, false, false, P, ld, P, ld, L + o1 * ld + o1, ld,
+                                        NB + rest, NB, NB, -1.0, true, false, KR_FULL, s));
+        GPK_TRY(launch_leaf_update(L, X, ld, o1, rest, leafinv + (o1 / NB) * NB * NB,
+                                   leafld + o1 / NB, leafinfo + o1 / NB, s));
+      }
+      return GPK_OK;
+    } else {
+      return potrf(0, n);
+    }
   }
   // Right-looking over panels of width B with a look-ahead of one panel: while
   // this stream applies panel j's update to the trailing columns beyond panel

@@ -233,6 +233,11 @@ template <typename TS>
 int launch_leaf(TS* A, TS* X, int64_t ld, int64_t o, double* leafinv, double* logdet, int* info,
                 const double* dsrc, hipStream_t s, const Batch& bt = Batch());
 
+// The float64 leaf at o >= NB together with the update C -= P P^T of the `rest` rows
+// and columns beyond it (lower NB-tiles) by the NB columns P before o.
+int launch_leaf_update(double* A, double* X, int64_t ld, int64_t o, int64_t rest,
+                       double* leafinv, double* logdet, int* info, hipStream_t s);
+
 // k-range modes of the tile GEMM.
 enum KRange { KR_FULL = 0, KR_GE_N = 1, KR_LE_M = 2, KR_GE_M = 3 };
 // Product arithmetic of the tile GEMM.  AR_FP16X3: float32 operands scaled by a

@@ -166,23 +166,22 @@ __device__ __forceinline__ void factor_panel(double* P, const double* ident, int
   }
 }
 
-template <typename TS>
-__global__ __launch_bounds__(LEAF_THREADS) void leaf_kernel(TS* A, TS* X, int64_t ld, int64_t o,
-                                                            double* __restrict__ leafinv,
-                                                            double* __restrict__ logdet,
-                                                            int* __restrict__ info,
-                                                            const double* __restrict__ dsrc,
-                                                            Batch bt) {
-  __shared__ double buf[2][PROWS * PLD];
-  __shared__ double ident[PB * PLD];
-  __shared__ double dk_s[NB];
-  A = bws(A, bt);
-  X = bws(X, bt);
-  leafinv = bws(leafinv, bt);
-  logdet = bws(logdet, bt);
-  info = bws(info, bt);
-  dsrc = bws(dsrc, bt);
+// LDS of one leaf.
+struct LeafShared {
+  double buf[2][PROWS * PLD];
+  double ident[PB * PLD];
+  double dk_s[NB];
+};
 
+// The leaf of the block at row and column o: the whole workgroup.
+template <typename TS>
+__device__ __forceinline__ void leaf_block(LeafShared& sh, TS* A, TS* X, int64_t ld, int64_t o,
+                                           double* __restrict__ leafinv,
+                                           double* __restrict__ logdet, int* __restrict__ info,
+                                           const double* __restrict__ dsrc) {
+  auto& buf = sh.buf;
+  auto& ident = sh.ident;
+  auto& dk_s = sh.dk_s;
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lr = lane >> 4, lc = lane & 15;  // accumulator element r: row lr + 4 r, column lc
@@ -308,6 +307,58 @@ __global__ __launch_bounds__(LEAF_THREADS) void leaf_kernel(TS* A, TS* X, int64_
   emit(NPAN - 1, buf[(NPAN - 1) & 1]);
 }
 
+template <typename TS>
+__global__ __launch_bounds__(LEAF_THREADS) void leaf_kernel(TS* A, TS* X, int64_t ld, int64_t o,
+                                                            double* __restrict__ leafinv,
+                                                            double* __restrict__ logdet,
+                                                            int* __restrict__ info,
+                                                            const double* __restrict__ dsrc,
+                                                            Batch bt) {
+  __shared__ LeafShared sh;
+  leaf_block(sh, bws(A, bt), bws(X, bt), ld, o, bws(leafinv, bt), bws(logdet, bt), bws(info, bt),
+             bws(dsrc, bt));
+}
+
+// The leaf at o (first workgroup) beside the update of the columns beyond it by the
+// solved panel before it (the others): C -= P P^T over the lower NB-tiles from row and
+// column o + NB on, P = the rows' NB columns before o.  One launch instead of two on
+// two streams, whose hand-over costs more than the leaf's dependents (see
+// Factor::potrf_steps).  A workgroup takes a 64 x 64 quarter of a tile, eight of its
+// waves 16 x 32 each straight from global memory.
+__global__ __launch_bounds__(LEAF_THREADS) void leaf_update_kernel(
+    double* A, double* X, int64_t ld, int64_t o, double* __restrict__ leafinv,
+    double* __restrict__ logdet, int* __restrict__ info) {
+  __shared__ LeafShared sh;
+  if (blockIdx.x == 0) {
+    leaf_block<double>(sh, A, X, ld, o, leafinv, logdet, info, nullptr);
+    return;
+  }
+  const int b = blockIdx.x - 1;
+  int64_t mt, nt;
+  lower_tile(b / 4, mt, nt);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  if (w >= 8) return;
+  const int64_t o2 = o + NB;
+  const int64_t mw = mt * NB + ((b >> 1) & 1) * 64 + (w >> 1) * 16;
+  const int64_t nw = nt * NB + (b & 1) * 64 + (w & 1) * 32;
+  const double* P = A + o2 * ld + o - NB;
+  double* C = A + o2 * ld + o2;
+  f64x4 acc[1][2];
+  DirectLoop<false, false, 1, 2> loop(P, ld, P, ld, mw, nw, lane, 0, NB);
+  const int lr = lane >> 4, lc = lane & 15;
+  double cv[2][4];
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) cv[j][r] = C[(mw + lr + 4 * r) * ld + nw + 16 * j + lc];
+  loop.run(acc);
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      C[(mw + lr + 4 * r) * ld + nw + 16 * j + lc] = cv[j][r] - acc[0][j][r];
+}
+
 }  // namespace
 
 template <typename TS>
@@ -315,6 +366,20 @@ int launch_leaf(TS* A, TS* X, int64_t ld, int64_t o, double* leafinv, double* lo
                 const double* dsrc, hipStream_t s, const Batch& bt) {
   hipLaunchKernelGGL(leaf_kernel<TS>, dim3(1, 1, bt.count), dim3(LEAF_THREADS), 0, s, A, X, ld,
                      o, leafinv, logdet, info, dsrc, bt);
+  GPK_LAUNCH_CHECK();
+  return GPK_OK;
+}
+
+int launch_leaf_update(double* A, double* X, int64_t ld, int64_t o, int64_t rest,
+                       double* leafinv, double* logdet, int* info, hipStream_t s) {
+  if (o < NB || rest < 0 || rest % NB) {
+    set_error("leaf update: block at %lld with %lld rows beyond it", (long long)o,
+              (long long)rest);
+    return GPK_ERR_BAD_ARG;
+  }
+  const int64_t T = rest / NB;
+  hipLaunchKernelGGL(leaf_update_kernel, dim3((unsigned)(1 + 2 * T * (T + 1))),
+                     dim3(LEAF_THREADS), 0, s, A, X, ld, o, leafinv, logdet, info);
   GPK_LAUNCH_CHECK();
   return GPK_OK;
 }
