@@ -359,6 +359,7 @@ __global__ __launch_bounds__(256, 2) void adjoint_small_kernel(
   double s_var = 0.0, s_tr = 0.0, s_ls[DMAX];
 #pragma unroll
   for (int q = 0; q < DMAX; ++q) s_ls[q] = 0.0;
+  with_kind(kind, [&](auto K) {
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -381,7 +382,7 @@ __global__ __launch_bounds__(256, 2) void adjoint_small_kernel(
           }
         }
         double kv, fv;
-        kval_fac(kind, d2, kv, fv);
+        kval_fac_of<K()>(d2, kv, fv);
         const double g = wt * wij;
         s_var += g * kv;
         if (gi == gj) s_tr += wij;
@@ -399,6 +400,7 @@ __global__ __launch_bounds__(256, 2) void adjoint_small_kernel(
         }
       }
     }
+  });
 #pragma unroll
   for (int q = 0; q < DMAX + 2; ++q) {
     double v = q < DMAX ? s_ls[q] : (q == DMAX ? s_var : s_tr);

@@ -1470,8 +1470,8 @@ int gpk_cross_covariance(int kind, const double* x, int64_t n, const double* z, 
     set_error("cross_covariance: bad z/out/m/ldo");
     return GPK_ERR_BAD_ARG;
   }
-  return launch_kernel_matrix<double>(kind, x, n, z, m, (int)d, theta, nls, 0.0, 0, out, ldo, n,
-                                      m, false, (hipStream_t)stream);
+  return launch_cross<double>(kind, x, n, z, m, (int)d, theta, nls, false, out, ldo, n, m,
+                              (hipStream_t)stream);
 }
 
 int gpk_gram(int kind, const double* x, int64_t n, int64_t d, const double* theta, int nls,
@@ -1482,6 +1482,10 @@ int gpk_gram(int kind, const double* x, int64_t n, int64_t d, const double* thet
     set_error("gram: bad out/ldo");
     return GPK_ERR_BAD_ARG;
   }
+  // no diagonal addition: the cross-covariance builder gives the same entries
+  if (jitter == 0.0 && !add_noise)
+    return launch_cross<double>(kind, x, n, x, n, (int)d, theta, nls, false, out, ldo, n, n,
+                                (hipStream_t)stream);
   return launch_kernel_matrix<double>(kind, x, n, x, n, (int)d, theta, nls, jitter,
                                       add_noise ? 2 : 1, out, ldo, n, n, false,
                                       (hipStream_t)stream);

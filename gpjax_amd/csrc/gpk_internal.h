@@ -103,7 +103,7 @@ __device__ __forceinline__ void bmember(const Batch& b, int d, PX& x, int64_t& n
 
 // ---------------------------------------------------------------------------
 // Stationary kernel formulas (unit variance), from rho^2 of the
-// lengthscale-scaled inputs.  kval() is k(rho); kfac() is F(rho) with
+// lengthscale-scaled inputs.  kval_of() is k(rho); kval_fac_of() also F(rho) with
 // dK/dl_d = var * F(rho) * u_d / l_d, u_d = (x_d - z_d)^2 / l_d^2.
 //   RBF        gpjax/kernels/stationary/rbf.py:43          k = exp(-rho^2/2)
 //   Matern-1/2 gpjax/kernels/stationary/matern12.py:47     k = exp(-rho)
@@ -111,11 +111,16 @@ __device__ __forceinline__ void bmember(const Batch& b, int d, PX& x, int64_t& n
 //   Matern-5/2 gpjax/kernels/stationary/matern52.py:47-52  k = (1+s5 rho+5/3 rho^2) exp(-s5 rho)
 // Matern distances are sqrt(max(rho^2, 1e-36)) (stationary/utils.py:67).
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ double kval(int kind, double d2) {
-  if (kind == GPK_KERNEL_RBF) return exp(-0.5 * d2);
+// The kernel kind is a template argument here: a switch per element puts every
+// exponential into a branch of its own, one dependent chain after the other with its
+// coefficients moved in again each time.  with_kind() takes the switch once around a
+// loop of elements, whose chains then overlap.
+template <int KIND>
+__device__ __forceinline__ double kval_of(double d2) {
+  if constexpr (KIND == GPK_KERNEL_RBF) return exp(-0.5 * d2);
   const double t = sqrt(fmax(d2, 1e-36));
-  if (kind == GPK_KERNEL_MATERN12) return exp(-t);
-  if (kind == GPK_KERNEL_MATERN32) {
+  if constexpr (KIND == GPK_KERNEL_MATERN12) return exp(-t);
+  if constexpr (KIND == GPK_KERNEL_MATERN32) {
     const double s3 = 1.7320508075688772;
     return (1.0 + s3 * t) * exp(-s3 * t);
   }
@@ -123,14 +128,15 @@ __device__ __forceinline__ double kval(int kind, double d2) {
   return (1.0 + s5 * t + (5.0 / 3.0) * t * t) * exp(-s5 * t);
 }
 
-// kval in float32 arithmetic (rho^2 formed in float64 by the caller), for
+// kval_of in float32 arithmetic (rho^2 formed in float64 by the caller), for
 // entries that are stored in float32 anyway: a few float32 ulps of relative
 // error instead of the half ulp of rounding a float64 value.
-__device__ __forceinline__ float kvalf(int kind, float d2) {
-  if (kind == GPK_KERNEL_RBF) return expf(-0.5f * d2);
+template <int KIND>
+__device__ __forceinline__ float kvalf_of(float d2) {
+  if constexpr (KIND == GPK_KERNEL_RBF) return expf(-0.5f * d2);
   const float t = sqrtf(fmaxf(d2, 1e-36f));
-  if (kind == GPK_KERNEL_MATERN12) return expf(-t);
-  if (kind == GPK_KERNEL_MATERN32) {
+  if constexpr (KIND == GPK_KERNEL_MATERN12) return expf(-t);
+  if constexpr (KIND == GPK_KERNEL_MATERN32) {
     const float s3 = 1.7320508f;
     return (1.0f + s3 * t) * expf(-s3 * t);
   }
@@ -139,57 +145,73 @@ __device__ __forceinline__ float kvalf(int kind, float d2) {
 }
 
 // Both k(rho) and F(rho) with one exponential.
-__device__ __forceinline__ void kval_fac(int kind, double d2, double& k, double& f) {
-  if (kind == GPK_KERNEL_RBF) {
+template <int KIND>
+__device__ __forceinline__ void kval_fac_of(double d2, double& k, double& f) {
+  if constexpr (KIND == GPK_KERNEL_RBF) {
     k = exp(-0.5 * d2);
     f = k;
     return;
   }
   const double t = sqrt(fmax(d2, 1e-36));
-  if (kind == GPK_KERNEL_MATERN12) {
+  if constexpr (KIND == GPK_KERNEL_MATERN12) {
     const double e = exp(-t);
     k = e;
     f = d2 > 1e-36 ? e / t : 0.0;
-    return;
-  }
-  if (kind == GPK_KERNEL_MATERN32) {
+  } else if constexpr (KIND == GPK_KERNEL_MATERN32) {
     const double s3 = 1.7320508075688772;
     const double e = exp(-s3 * t);
     k = (1.0 + s3 * t) * e;
     f = 3.0 * e;
-    return;
+  } else {
+    const double s5 = 2.23606797749979;
+    const double e = exp(-s5 * t);
+    k = (1.0 + s5 * t + (5.0 / 3.0) * t * t) * e;
+    f = (5.0 / 3.0) * (1.0 + s5 * t) * e;
   }
-  const double s5 = 2.23606797749979;
-  const double e = exp(-s5 * t);
-  k = (1.0 + s5 * t + (5.0 / 3.0) * t * t) * e;
-  f = (5.0 / 3.0) * (1.0 + s5 * t) * e;
 }
 
-// kval_fac in float32 arithmetic (the mixed collapsed ELBO's gradient pass).
-__device__ __forceinline__ void kval_facf(int kind, float d2, float& k, float& f) {
-  if (kind == GPK_KERNEL_RBF) {
+// kval_fac_of in float32 arithmetic (the mixed collapsed ELBO's gradient pass).
+template <int KIND>
+__device__ __forceinline__ void kval_facf_of(float d2, float& k, float& f) {
+  if constexpr (KIND == GPK_KERNEL_RBF) {
     k = expf(-0.5f * d2);
     f = k;
     return;
   }
   const float t = sqrtf(fmaxf(d2, 1e-36f));
-  if (kind == GPK_KERNEL_MATERN12) {
+  if constexpr (KIND == GPK_KERNEL_MATERN12) {
     const float e = expf(-t);
     k = e;
     f = d2 > 1e-36f ? e / t : 0.0f;
-    return;
-  }
-  if (kind == GPK_KERNEL_MATERN32) {
+  } else if constexpr (KIND == GPK_KERNEL_MATERN32) {
     const float s3 = 1.7320508f;
     const float e = expf(-s3 * t);
     k = (1.0f + s3 * t) * e;
     f = 3.0f * e;
-    return;
+  } else {
+    const float s5 = 2.2360680f;
+    const float e = expf(-s5 * t);
+    k = (1.0f + s5 * t + (5.0f / 3.0f) * t * t) * e;
+    f = (5.0f / 3.0f) * (1.0f + s5 * t) * e;
   }
-  const float s5 = 2.2360680f;
-  const float e = expf(-s5 * t);
-  k = (1.0f + s5 * t + (5.0f / 3.0f) * t * t) * e;
-  f = (5.0f / 3.0f) * (1.0f + s5 * t) * e;
+}
+
+// f(std::integral_constant<int, kind>()).
+template <typename F>
+__device__ __forceinline__ void with_kind(int kind, F&& f) {
+  if (kind == GPK_KERNEL_RBF) f(std::integral_constant<int, GPK_KERNEL_RBF>());
+  else if (kind == GPK_KERNEL_MATERN12) f(std::integral_constant<int, GPK_KERNEL_MATERN12>());
+  else if (kind == GPK_KERNEL_MATERN32) f(std::integral_constant<int, GPK_KERNEL_MATERN32>());
+  else f(std::integral_constant<int, GPK_KERNEL_MATERN52>());
+}
+
+// By runtime kind, for loops that one element at a time is enough for (the collapsed
+// ELBO's data pass, with 2 d + 1 sums per thread: a kernel per kind was no faster).
+__device__ __forceinline__ void kval_fac(int kind, double d2, double& k, double& f) {
+  with_kind(kind, [&](auto K) { kval_fac_of<K()>(d2, k, f); });
+}
+__device__ __forceinline__ void kval_facf(int kind, float d2, float& k, float& f) {
+  with_kind(kind, [&](auto K) { kval_facf_of<K()>(d2, k, f); });
 }
 
 // ---------------------------------------------------------------------------

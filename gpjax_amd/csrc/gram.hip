@@ -99,13 +99,17 @@ __global__ __launch_bounds__(256) void kmat_kernel(int kind, const double* __res
   const double sd = theta[nls + 1];
   const int64_t j = j0 + jj;
   if (j >= cols_total) return;
+  with_kind(kind, [&](auto K) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) d2[r] = var * kval_of<K()>(d2[r]);
+  });
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int64_t i = i0 + rg * 16 + r;
     if (i >= rows_total) continue;
     double v;
     if (i < n && j < m) {
-      v = var * kval(kind, d2[r]);
+      v = d2[r];
       const int dm = diag_mode & KM_DIAG_MASK;
       if (dm > 0 && i == j) {
         v = v + jitter;
@@ -130,25 +134,27 @@ __global__ __launch_bounds__(256) void kmat_kernel(int kind, const double* __res
 // Cross-covariance over a long stream of points (the collapsed ELBO's Kzx
 // chunks): out[i][j] = var k(x_i / l, z_j / l) for i < n, j < m, zero elsewhere
 // up to rows_total x cols_total.  One 256-thread block owns 64 rows (x, scaled
-// and staged once in LDS, read as wave-wide broadcasts) and walks CT column
-// tiles of 64 (z) through two LDS buffers: the next tile's scaled inputs are
+// and staged once in LDS, read as wave-wide broadcasts) and walks `ct` column
+// tiles of 64 (z; CT, or fewer until the grid has 1,024 blocks) through two LDS buffers: the next tile's scaled inputs are
 // loaded into registers before the current tile's arithmetic and stored after
 // it, so their global-load latency hides behind a tile of work.  Thread
 // (rg, jj) = (wave, lane) computes rows rg*16 .. +15 of column jj.  kmat_kernel's
 // short-lived blocks (one tile, inputs staged per tile) ran at a third of the
 // store and ALU bound on these shapes.  The dimension loop stays a runtime loop
 // (unrolled, the compiler issues all 16 x d row reads at once and runs out of
-// registers).  The distances are the same arithmetic in the same order as
+// registers); the kernel function runs over the thread's 16 entries in one block per
+// kind (with_kind), so their exponentials overlap
+// (10,007 x 4,099, d = 8, float64: kmat_kernel 158 us, 109 us here).  The distances are the same arithmetic in the same order as
 // kmat_kernel's, so the float64 entries are identical; F32K evaluates the
-// kernel function in float32 (kvalf).
-constexpr int CT = 8;
+// kernel function in float32 (kvalf_of).
+constexpr int CT = 8;  // most column tiles per block
 
 template <typename TS, bool F32K, int DMAX>
 __global__ __launch_bounds__(256) void cross_kernel(int kind, const double* __restrict__ x,
                                                     int64_t n, const double* __restrict__ z,
                                                     int64_t m, int d,
                                                     const double* __restrict__ theta, int nls,
-                                                    TS* __restrict__ out, int64_t ldo,
+                                                    int ct, TS* __restrict__ out, int64_t ldo,
                                                     int64_t rows_total, int64_t cols_total) {
   constexpr int NPRE = KT * DMAX / 256;  // staged inputs per thread and tile (DMAX >= 4)
   __shared__ double xs[DMAX][KT];  // [dimension][row]: a wave's 16 rows are contiguous
@@ -179,13 +185,13 @@ __global__ __launch_bounds__(256) void cross_kernel(int kind, const double* __re
     }
   };
   const int64_t ntiles = (cols_total + KT - 1) / KT;
-  int64_t jt = (int64_t)blockIdx.x * CT;
+  int64_t jt = (int64_t)blockIdx.x * ct;
   load(jt);
   stage(0);
   const double var = theta[nls];
   __syncthreads();
-  for (int c = 0; c < CT && jt < ntiles; ++c, ++jt) {
-    const bool more = c + 1 < CT && jt + 1 < ntiles;
+  for (int c = 0; c < ct && jt < ntiles; ++c, ++jt) {
+    const bool more = c + 1 < ct && jt + 1 < ntiles;
     if (more) load(jt + 1);
     const int b = c & 1;
     double d2[16];
@@ -199,18 +205,24 @@ __global__ __launch_bounds__(256) void cross_kernel(int kind, const double* __re
         d2[r] += df * df;
       }
     }
+    TS kv[16];
+    with_kind(kind, [&](auto K) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        if constexpr (F32K) kv[r] = (float)var * kvalf_of<K()>((float)d2[r]);
+        else kv[r] = (TS)(var * kval_of<K()>(d2[r]));
+      }
+    });
     const int64_t j = jt * KT + jj;
-    if (j < cols_total) {
+    TS* o = out + (i0 + rg * 16) * ldo + j;
+    if (i0 + KT <= n && (jt + 1) * KT <= m) {  // the whole tile is inside
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[r * ldo] = kv[r];
+    } else if (j < cols_total) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int64_t i = i0 + rg * 16 + r;
-        if (i >= rows_total) break;
-        const bool in = i < n && j < m;
-        if constexpr (F32K) {
-          out[i * ldo + j] = in ? (float)var * kvalf(kind, (float)d2[r]) : 0.0f;
-        } else {
-          out[i * ldo + j] = (TS)(in ? var * kval(kind, d2[r]) : 0.0);
-        }
+        if (i < rows_total) o[r * ldo] = i < n && j < m ? kv[r] : (TS)0;
       }
     }
     if (more) stage(b ^ 1);
@@ -239,16 +251,18 @@ int launch_cross(int kind, const double* x, int64_t n, const double* z, int64_t 
     return GPK_ERR_BAD_ARG;
   }
   const int64_t ntiles = (cols_total + KT - 1) / KT;
-  dim3 grid((unsigned)((ntiles + CT - 1) / CT), (unsigned)gy, 1);
+  int ct = CT;
+  while (ct > 1 && (ntiles + ct - 1) / ct * gy < 1024) ct /= 2;
+  dim3 grid((unsigned)((ntiles + ct - 1) / ct), (unsigned)gy, 1);
 #define GPK_CROSS(DM)                                                                          \
   do {                                                                                         \
     if (f32k)                                                                                  \
       hipLaunchKernelGGL((cross_kernel<TS, std::is_same<TS, float>::value, DM>), grid,         \
-                         dim3(256), 0, s, kind, x, n, z, m, d, theta, nls, out, ldo,           \
+                         dim3(256), 0, s, kind, x, n, z, m, d, theta, nls, ct, out, ldo,       \
                          rows_total, cols_total);                                              \
     else                                                                                       \
       hipLaunchKernelGGL((cross_kernel<TS, false, DM>), grid, dim3(256), 0, s, kind, x, n, z, \
-                         m, d, theta, nls, out, ldo, rows_total, cols_total);                  \
+                         m, d, theta, nls, ct, out, ldo, rows_total, cols_total);              \
   } while (0)
   if (d <= 4) GPK_CROSS(4);
   else if (d <= 8) GPK_CROSS(8);

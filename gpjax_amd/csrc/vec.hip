@@ -225,8 +225,12 @@ __global__ __launch_bounds__(256) void sigma_mv_kernel(int kind, const double* _
             const double df = xi[q] - xj_s[jj + u][q];
             d2 += df * df;
           }
-          kv[u] = var * kval(kind, d2);
+          kv[u] = d2;
         }
+        with_kind(kind, [&](auto K) {
+#pragma unroll
+          for (int u = 0; u < SMV_U; ++u) kv[u] = var * kval_of<K()>(kv[u]);
+        });
 #pragma unroll
         for (int u = 0; u < SMV_U; ++u)
 #pragma unroll
