@@ -6,8 +6,10 @@
 //      leaves multiply by the float64 leaf inverses); A22 -= L21 L21^T (SYRK on
 //      the matrix cores); potrf(A22).  Leaves factor NB x NB blocks in float64
 //      and also emit their inverses and log-diagonal sums.  Single problems of
-//      at least four 2,048-wide panels take the look-ahead form (factor.h).
-//   3. Recursive triangular inverse X = L^-1:  X21 = -X22 (L21 X11).
+//      more than 4,096 rows (float32 storage: 2,048 on) take the look-ahead form,
+//      smaller float64 ones go leaf by leaf (factor.h).
+//   3. Recursive triangular inverse X = L^-1:  X21 = -X22 (L21 X11); leaf by leaf it
+//      comes with step 2.
 //   4. alpha = X^T X r, then float64 iterative refinement against Sigma in
 //      float64 (a stored copy in the mixed path, recomputed from the inputs in
 //      the FP64 path): alpha += X^T X (r - Sigma alpha), stopped on the device
@@ -687,11 +689,13 @@ int mll_forward_t(int kind, const Arith3& ar, const double* x, const double* y, 
                                      true, s, dblk, bt, spk));
   }
   {
+    // (the inverse of a small float64 problem comes with its factor)
     PhaseScope ps(GPK_PHASE_POTRF, s);
     if (bt.gp) GPK_TRY(F.potrf(0, np));
-    else GPK_TRY(F.factor(np, true));
+    else if (f64 && np <= STEPS_MAX) GPK_TRY(F.potrf_steps(np, true));
+    else GPK_TRY(F.factor_only(np, true));
   }
-  {
+  if (bt.gp || !f64 || np > STEPS_MAX) {
     PhaseScope ps(GPK_PHASE_TRTRI, s);
     GPK_TRY(F.trtri(0, np));
   }

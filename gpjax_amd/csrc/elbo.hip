@@ -828,8 +828,7 @@ int elbo_forward_impl(int kind, const ElboArith& ea, const double* x, const doub
     FK.s = s2;
     GPK_TRY(launch_kernel_matrix<double>(kind, z, m, z, m, d, theta, nls, jitter, 1, Kb, mp, mp,
                                          mp, true, s2));
-    GPK_TRY(FK.factor(mp, false));
-    GPK_TRY(FK.trtri(0, mp));
+    GPK_TRY(FK.factor(mp, false, true));
     GPK_TRY(launch_gemm<double, double, double>(AR_F64, true, true, FK.X, mp, FK.X, mp, Kinv, mp,
                                                 mp, mp, mp, 1.0, false, true, KR_GE_M, s2));
     hipLaunchKernelGGL(mirror_kernel, dim3(cdiv(mp * mp, 256)), dim3(256), 0, s2, Kinv, mp, mp);
@@ -877,8 +876,7 @@ int elbo_forward_impl(int kind, const ElboArith& ea, const double* x, const doub
   Factor<double> FC{Cb, at<double>(ws, Lo.off_XC), mp, T, at<double>(ws, Lo.off_liC),
                     at<double>(ws, Lo.off_ldC), at<int>(ws, Lo.off_ifC), AR_F64, AR_F64, s};
   // The Kzz branch has joined, so the look-ahead's second stream is free here.
-  GPK_TRY(FC.factor(mp, true));
-  GPK_TRY(FC.trtri(0, mp));
+  GPK_TRY(FC.factor(mp, true, true));
   // 3. c = C^-1 b = X_C^T X_C b
   GPK_TRY(launch_trmv<double>(FC.X, mp, mp, b, u, false, vpart, s));
   GPK_TRY(launch_trmv<double>(FC.X, mp, mp, u, cvec, true, vpart, s));

@@ -5,6 +5,8 @@
 //   trsm(B, L): Y L^T = B by recursion on the columns, leaves multiplying by the
 //               float64 inverse of an NB x NB diagonal block
 //   trtri(L):   X = L^-1 with X21 = -X22 (L21 X11), both halves recursively
+// A single float64 problem up to STEPS_MAX rows instead goes leaf by leaf, factor and
+// inverse in one sweep (Factor::potrf_steps); larger single problems go by panels.
 // These replace jnp.linalg.cholesky, jsp.linalg.solve_triangular and the
 // LU-based slogdet/solve behind gpjax/linalg/operations.py:54-55,105-111,163-165.
 // Splits fall on multiples of NB; leaves (NB x NB) are factored and inverted
@@ -32,8 +34,9 @@ constexpr unsigned TRI_NODEWISE = 64;  // members from which the inverse goes no
 // Largest single float64 problem factored leaf by leaf on one stream
 // (Factor::potrf_steps).  Beyond it the trailing updates, a rank-128 step each, take
 // longer than the leaf they run beside.  MLL + gradient (two streams with the
-// look-ahead / leaf by leaf, ms): n = 2,000 1.41 / 1.04, n = 3,001 (leave-one-out)
-// 3.16 / 2.67, n = 4,000 3.80 / 3.37, n = 6,000 8.5 / 8.7, n = 8,000 15.6 / 17.3.
+// look-ahead / leaf by leaf with the inverse in the sweep, ms): n = 2,000 1.41 / 0.85,
+// n = 3,001 (leave-one-out) 3.16 / 2.42, n = 4,000 3.80 / 3.25; with the inverse after
+// the factor on both sides: n = 6,000 8.5 / 8.7, n = 8,000 15.6 / 17.3.
 constexpr int64_t STEPS_MAX = 4096;
 
 // Panel width of the look-ahead Cholesky (Factor::potrf_lookahead) for a single
@@ -160,27 +163,37 @@ struct Factor {
                                     dblk_at(o + h), bt, fscale));
     return potrf(o + h, n - h);
   }
-  // The whole factorisation of one problem (no batch).  `streams`: the look-ahead may
-  // use this thread's second stream.
-  int factor(int64_t n, bool streams) {
+  // The whole factorisation of one problem (no batch); `inverse`: X = L^-1 too.
+  // `streams`: the look-ahead may use this thread's second stream.
+  int factor(int64_t n, bool streams, bool inverse) {
     const bool f32 = std::is_same<TS, float>::value;
-    if (!f32 && n <= STEPS_MAX) return potrf_steps(n);
-    const int64_t la = streams ? lookahead_width(n, f32) : 0;
+    if (!f32 && n <= STEPS_MAX) return potrf_steps(n, inverse);
+    GPK_TRY(factor_only(n, streams));
+    return inverse ? trtri(0, n) : GPK_OK;
+  }
+  int factor_only(int64_t n, bool streams) {
+    const int64_t la = streams ? lookahead_width(n, std::is_same<TS, float>::value) : 0;
     return la > 0 ? potrf_lookahead(n, la) : potrf(0, n);
   }
-  // Right-looking in single leaves on one stream (float64): per leaf a launch of the
-  // leaf beside the trailing update by the panel before it, one of the column block's
-  // solve, and one of the next column block's update.
-  int potrf_steps(int64_t n) {
+  // Right-looking in single leaves on one stream (float64), the factor and, with
+  // `inverse`, its inverse in one sweep.  Per leaf, three launches: the solve of the
+  // column block below it and of the inverse's row block left of it; the next column
+  // block's update; the next leaf beside everything else that panel updates.
+  // The inverse's products fill CUs that the leaf leaves idle: the value and gradient
+  // with the inverse after the factor, level by level, 1,026 us at n = 2,000 and 3,393 at
+  // 4,000; in the sweep 852 and 3,245.
+  int potrf_steps(int64_t n, bool inverse) {
     if constexpr (std::is_same<TS, double>::value) {
       GPK_TRY(leaf(0));
-      for (int64_t o = 0; o + NB < n; o += NB) {
+      for (int64_t o = 0; o < n; o += NB) {
         const int64_t o1 = o + NB, rest = n - o1 - NB;
-        GPK_TRY(trsm(o1, n - o1, o, NB));
+        GPK_TRY(launch_step_solve(L + o1 * ld + o, X + o * ld, ld, n - o1, inverse ? o : 0,
+                                  leafinv + (o / NB) * NB * NB, s));
+        if (o1 == n) break;
         const TS* P = L + o1 * ld + o;
         GPK_TRY(launch_gemm<TS, TS, TS>(AR_F64, false, false, P, ld, P, ld, L + o1 * ld + o1, ld,
                                         NB + rest, NB, NB, -1.0, true, false, KR_FULL, s));
-        GPK_TRY(launch_leaf_update(L, X, ld, o1, rest, leafinv + (o1 / NB) * NB * NB,
+        GPK_TRY(launch_leaf_update(L, X, ld, o1, rest, inverse, leafinv + (o1 / NB) * NB * NB,
                                    leafld + o1 / NB, leafinfo + o1 / NB, s));
       }
       return GPK_OK;

@@ -237,15 +237,11 @@ int launch_small(bool a_km, bool b_kn, const GemmParams& p, hipStream_t s) {
 // computes column blocks w and 7 - w (of 16), k only up to the diagonal, so every
 // wave issues nine slabs.  15 blocks of 128 rows: 24 us as 128 x 128 tiles, 7 us.
 template <int MI>
-__global__ __launch_bounds__(256) void trsm_strip_kernel(double* B, int64_t ld,
-                                                         const double* __restrict__ inv,
-                                                         Batch bt) {
+__device__ __forceinline__ void trsm_strip(double* B, int64_t ld, const double* __restrict__ inv,
+                                           int64_t r0) {
   constexpr int NS = NB / SLAB;
-  B = bws(B, bt);
-  inv = bws(inv, bt);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int lr = lane >> 4, lc = lane & 15;
-  const int64_t r0 = (int64_t)blockIdx.x * 16 * MI;
   double av[NS][MI][4], bv[NS + 1][4];
 #pragma unroll
   for (int s = 0; s < NS; ++s)
@@ -291,6 +287,63 @@ __global__ __launch_bounds__(256) void trsm_strip_kernel(double* B, int64_t ld,
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         B[(r0 + 16 * i + lr + 4 * r) * ld + (c ? w : NS - 1 - w) * 16 + lc] = acc[c][i][r];
+}
+
+template <int MI>
+__global__ __launch_bounds__(256) void trsm_strip_kernel(double* B, int64_t ld,
+                                                         const double* __restrict__ inv,
+                                                         Batch bt) {
+  trsm_strip<MI>(bws(B, bt), ld, bws(inv, bt), (int64_t)blockIdx.x * 16 * MI);
+}
+
+// X = L11^-1 N in place for the 16 columns from c0 of NB rows (the same roles with the
+// inverse on the left): wave w computes row blocks w and 7 - w.
+__device__ __forceinline__ void inverse_strip(double* N, int64_t ld,
+                                              const double* __restrict__ inv, int64_t c0) {
+  constexpr int NS = NB / SLAB;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lr = lane >> 4, lc = lane & 15;
+  double av[NS + 1][4], bv[NS][4];
+#pragma unroll
+  for (int s = 0; s < NS; ++s) frag_load<true>(N, ld, c0 + lc, s * SLAB + 4 * lr, bv[s]);
+#pragma unroll
+  for (int t = 0; t <= NS; ++t) {
+    const int second = t >= NS - w;
+    const int I = second ? w : NS - 1 - w, s = second ? t - (NS - w) : t;
+    frag_load<false>(inv, NB, I * 16 + lc, s * SLAB + 4 * lr, av[t]);
+  }
+  __syncthreads();
+  f64x4 acc[2] = {f64x4{0.0, 0.0, 0.0, 0.0}, f64x4{0.0, 0.0, 0.0, 0.0}};
+  auto products = [&](auto wc) {
+    constexpr int split = NS - decltype(wc)::value;
+#pragma unroll
+    for (int t = 0; t <= NS; ++t) {
+      const int c = t >= split ? 1 : 0, s = t >= split ? t - split : t;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[t][q], bv[s][q], acc[c], 0, 0, 0);
+    }
+  };
+  if (w == 0) products(std::integral_constant<int, 0>());
+  else if (w == 1) products(std::integral_constant<int, 1>());
+  else if (w == 2) products(std::integral_constant<int, 2>());
+  else products(std::integral_constant<int, 3>());
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      N[((c ? w : NS - 1 - w) * 16 + lr + 4 * r) * ld + c0 + lc] = acc[c][r];
+}
+
+// What follows a leaf whose inverse is `inv`: the solve of the column block B below it
+// (`rows` rows, the first rows / 16 workgroups) and the inverse's row block N left of
+// it (`cols` columns, the others).
+__global__ __launch_bounds__(256) void step_solve_kernel(double* B, double* N, int64_t ld,
+                                                         const double* __restrict__ inv,
+                                                         int64_t rows) {
+  const int64_t nb = rows / 16;
+  if (blockIdx.x < nb) trsm_strip<1>(B, ld, inv, (int64_t)blockIdx.x * 16);
+  else inverse_strip(N, ld, inv, ((int64_t)blockIdx.x - nb) * 16);
 }
 
 template <int AR, typename TA, typename TB, typename TC, bool A_KM, bool B_KN>
@@ -388,6 +441,20 @@ template int launch_tri_level<double>(int, const TriLevel&, int64_t, int64_t, co
 template int launch_tri_level<float>(int, const TriLevel&, int64_t, int64_t, const float*,
                                      int64_t, const float*, int64_t, float*, int64_t, hipStream_t,
                                      const Batch&, const float*);
+
+int launch_step_solve(double* B, double* N, int64_t ld, int64_t rows, int64_t cols,
+                      const double* inv, hipStream_t s) {
+  if (rows + cols <= 0) return GPK_OK;
+  if (rows % NB || cols % NB) {
+    set_error("step solve: %lld rows, %lld columns not multiples of %d", (long long)rows,
+              (long long)cols, NB);
+    return GPK_ERR_BAD_ARG;
+  }
+  hipLaunchKernelGGL(step_solve_kernel, dim3((unsigned)((rows + cols) / 16)), dim3(256), 0, s, B,
+                     N, ld, inv, rows);
+  GPK_LAUNCH_CHECK();
+  return GPK_OK;
+}
 
 int launch_trsm_strip(double* B, int64_t ld, int64_t m, const double* inv, hipStream_t s,
                       const Batch& bt) {

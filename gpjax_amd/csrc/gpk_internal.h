@@ -256,9 +256,14 @@ int launch_leaf(TS* A, TS* X, int64_t ld, int64_t o, double* leafinv, double* lo
                 const double* dsrc, hipStream_t s, const Batch& bt = Batch());
 
 // The float64 leaf at o >= NB together with the update C -= P P^T of the `rest` rows
-// and columns beyond it (lower NB-tiles) by the NB columns P before o.
-int launch_leaf_update(double* A, double* X, int64_t ld, int64_t o, int64_t rest,
+// and columns beyond it (lower NB-tiles) by the NB columns P before o and, with
+// `inverse`, of the unfinished rows of the inverse by the finished row before o.
+int launch_leaf_update(double* A, double* X, int64_t ld, int64_t o, int64_t rest, bool inverse,
                        double* leafinv, double* logdet, int* info, hipStream_t s);
+// After a leaf with inverse `inv`: B (`rows` x NB) <- B inv^T and N (NB x `cols`) <-
+// inv N, both in place.
+int launch_step_solve(double* B, double* N, int64_t ld, int64_t rows, int64_t cols,
+                      const double* inv, hipStream_t s);
 
 // k-range modes of the tile GEMM.
 enum KRange { KR_FULL = 0, KR_GE_N = 1, KR_LE_M = 2, KR_GE_M = 3 };
@@ -430,8 +435,8 @@ int launch_sigma_matvec(int kind, const double* x, int64_t n, int64_t np, int d,
 // calling thread on the current device, created on first use and kept for the
 // process.  The look-ahead Cholesky takes stream 0 and events 0..2 (never
 // inside a batched call); the batched driver takes the streams and events
-// 3..3+AUX_STREAMS; the collapsed ELBO takes stream 0 and events 6 and 7 (it
-// never runs the look-ahead Cholesky).
+// 3..3+AUX_STREAMS; the collapsed ELBO takes stream 0 and events 6 and 7
+// (joined before its M x M factor, which alone may run the look-ahead Cholesky).
 constexpr int AUX_STREAMS = 3;
 constexpr int AUX_EVENTS = 8;
 int aux_streams(hipStream_t* streams, hipEvent_t* events);

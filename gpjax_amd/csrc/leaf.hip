@@ -319,39 +319,60 @@ __global__ __launch_bounds__(LEAF_THREADS) void leaf_kernel(TS* A, TS* X, int64_
              bws(dsrc, bt));
 }
 
-// The leaf at o (first workgroup) beside the update of the columns beyond it by the
-// solved panel before it (the others): C -= P P^T over the lower NB-tiles from row and
-// column o + NB on, P = the rows' NB columns before o.  One launch instead of two on
-// two streams, whose hand-over costs more than the leaf's dependents (see
-// Factor::potrf_steps).  A workgroup takes a 64 x 64 quarter of a tile, eight of its
-// waves 16 x 32 each straight from global memory.
+// The leaf at o (first workgroup) beside the updates by the solved panel before it, P =
+// the NB columns before o (the others): C -= P P^T over the lower NB-tiles from row and
+// column o + NB on and, with `inverse`, the rows of the inverse not yet finished:
+// X[J][I] -= L[J][p] X[p][I] for every block row J >= o / NB and column I <= p =
+// o / NB - 1 (X[J][p] starts here: it is written without being read).  One launch
+// instead of several on two streams, whose hand-over costs more than the leaf's
+// dependents (see Factor::potrf_steps).  A workgroup takes a 64 x 64 quarter of a tile,
+// eight of its waves 16 x 32 each straight from global memory.
 __global__ __launch_bounds__(LEAF_THREADS) void leaf_update_kernel(
-    double* A, double* X, int64_t ld, int64_t o, double* __restrict__ leafinv,
-    double* __restrict__ logdet, int* __restrict__ info) {
+    double* A, double* X, int64_t ld, int64_t o, int64_t trailing, int inverse,
+    double* __restrict__ leafinv, double* __restrict__ logdet, int* __restrict__ info) {
   __shared__ LeafShared sh;
   if (blockIdx.x == 0) {
     leaf_block<double>(sh, A, X, ld, o, leafinv, logdet, info, nullptr);
     return;
   }
-  const int b = blockIdx.x - 1;
-  int64_t mt, nt;
-  lower_tile(b / 4, mt, nt);
+  int b = blockIdx.x - 1;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   if (w >= 8) return;
-  const int64_t o2 = o + NB;
-  const int64_t mw = mt * NB + ((b >> 1) & 1) * 64 + (w >> 1) * 16;
-  const int64_t nw = nt * NB + (b & 1) * 64 + (w & 1) * 32;
-  const double* P = A + o2 * ld + o - NB;
-  double* C = A + o2 * ld + o2;
-  f64x4 acc[1][2];
-  DirectLoop<false, false, 1, 2> loop(P, ld, P, ld, mw, nw, lane, 0, NB);
+  const int64_t ms = ((b >> 1) & 1) * 64 + (w >> 1) * 16, ns = (b & 1) * 64 + (w & 1) * 32;
   const int lr = lane >> 4, lc = lane & 15;
+  b /= 4;
+  f64x4 acc[1][2];
   double cv[2][4];
+  double* C;
+  int64_t mw, nw;
+  auto fetch = [&](bool read) {
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) cv[j][r] = C[(mw + lr + 4 * r) * ld + nw + 16 * j + lc];
-  loop.run(acc);
+      for (int r = 0; r < 4; ++r)
+        cv[j][r] = read ? C[(mw + lr + 4 * r) * ld + nw + 16 * j + lc] : 0.0;
+  };
+  if (b < trailing) {
+    int64_t mt, nt;
+    lower_tile(b, mt, nt);
+    mw = mt * NB + ms;
+    nw = nt * NB + ns;
+    const double* P = A + (o + NB) * ld + o - NB;
+    C = A + (o + NB) * ld + o + NB;
+    DirectLoop<false, false, 1, 2> loop(P, ld, P, ld, mw, nw, lane, 0, NB);
+    fetch(true);
+    loop.run(acc);
+  } else {
+    const int p = (int)(o / NB) - 1, q = b - (int)trailing;
+    const int J = q / (p + 1), I = q % (p + 1);
+    mw = J * NB + ms;
+    nw = I * NB + ns;
+    C = X + o * ld;
+    DirectLoop<false, true, 1, 2> loop(A + o * ld + o - NB, ld, X + (o - NB) * ld, ld, mw, nw,
+                                       lane, 0, NB);
+    fetch(I < p);
+    loop.run(acc);
+  }
 #pragma unroll
   for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -370,16 +391,18 @@ int launch_leaf(TS* A, TS* X, int64_t ld, int64_t o, double* leafinv, double* lo
   return GPK_OK;
 }
 
-int launch_leaf_update(double* A, double* X, int64_t ld, int64_t o, int64_t rest,
+int launch_leaf_update(double* A, double* X, int64_t ld, int64_t o, int64_t rest, bool inverse,
                        double* leafinv, double* logdet, int* info, hipStream_t s) {
-  if (o < NB || rest < 0 || rest % NB) {
+  if (o < NB || o % NB || rest < 0 || rest % NB) {
     set_error("leaf update: block at %lld with %lld rows beyond it", (long long)o,
               (long long)rest);
     return GPK_ERR_BAD_ARG;
   }
-  const int64_t T = rest / NB;
-  hipLaunchKernelGGL(leaf_update_kernel, dim3((unsigned)(1 + 2 * T * (T + 1))),
-                     dim3(LEAF_THREADS), 0, s, A, X, ld, o, leafinv, logdet, info);
+  const int64_t T = rest / NB, trailing = T * (T + 1) / 2;
+  const int64_t inv = inverse ? (T + 1) * (o / NB) : 0;
+  hipLaunchKernelGGL(leaf_update_kernel, dim3((unsigned)(1 + 4 * (trailing + inv))),
+                     dim3(LEAF_THREADS), 0, s, A, X, ld, o, trailing, inverse ? 1 : 0, leafinv,
+                     logdet, info);
   GPK_LAUNCH_CHECK();
   return GPK_OK;
 }

@@ -262,7 +262,7 @@ int potrf_t(int prec, const double* A, int64_t n, int64_t lda, double* Lout, int
                s};
   F.dblk = dblk;
   (void)prec;
-  GPK_TRY(F.factor(np, false));
+  GPK_TRY(F.factor(np, false, false));
   hipLaunchKernelGGL(store_kernel<TS>, dim3((unsigned)((n + 255) / 256), rows_grid(n)),
                      dim3(256), 0, s, L, np, n, 0, Lout, ldl);
   GPK_LAUNCH_CHECK();
@@ -435,8 +435,7 @@ int gpk_mvn_log_prob(const double* loc, const double* S, int64_t n, int64_t lds,
                    (int)AR_F64,
                    (int)AR_F64,
                    s};
-  GPK_TRY(F.factor(np, false));
-  GPK_TRY(F.trtri(0, np));
+  GPK_TRY(F.factor(np, false, true));
   hipLaunchKernelGGL(potrf_finish_kernel, dim3(1), dim3(64), 0, s, at<double>(ws, P.off_leafld),
                      at<int>(ws, P.off_leafinfo), nt, ldv, nullptr);
   GPK_LAUNCH_CHECK();

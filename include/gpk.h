@@ -17,8 +17,8 @@
  *     through `prec`.
  *   - Some calls fork work onto those library streams and join it back into
  *     `stream` with events before they return (the look-ahead Cholesky for
- *     n > 1,920, and for the collapsed ELBO's M x M factor when m > 1,920, the
- *     batched size buckets, the collapsed ELBO's Kzz-side work during its
+ *     n > 4,096 in float64 and n > 1,920 in the mixed precisions, also for the
+ *     collapsed ELBO's M x M factor when m > 4,096, the batched size buckets, the collapsed ELBO's Kzz-side work during its
  *     streamed chunks): to the caller the call stays
  *     ordered on `stream`, and under HIP-graph capture the fork and join become
  *     graph edges.  The streams and events are created by a thread's first
@@ -456,7 +456,7 @@ int gpk_adam_step(int64_t count, const double* grad, const uint8_t* softplus_mas
  */
 #define GPK_PHASE_GRAM 0    /* Sigma assembly                                  */
 #define GPK_PHASE_POTRF 1   /* recursive Cholesky (leaves, TRSM, SYRK)          */
-#define GPK_PHASE_TRTRI 2   /* recursive triangular inverse                    */
+#define GPK_PHASE_TRTRI 2   /* triangular inverse (float64, n <= 4,096: in POTRF)  */
 #define GPK_PHASE_SOLVE 3   /* alpha, float64 refinement, log-det, objective    */
 #define GPK_PHASE_ADJOINT 4 /* fused Sigma^-1 + gradient pass (backward)        */
 #define GPK_PHASE_COUNT 5

@@ -1,0 +1,137 @@
+"""Edges of the rules that pick a kernel by size: each route against the float64 oracle
+or against the general path.
+
+One leaf (n <= 128) with d <= 16 ends in a single launch, d = 17 in the general
+launches; float64 problems padded to at most 4,096 rows are factored leaf by leaf with
+the inverse in the same sweep, larger ones by panels with the inverse afterwards; kernel
+matrices take one builder whose tiles are cut at ragged edges; the collapsed ELBO splits
+odd chunk widths over the chip.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+import gpjax_amd as gpx
+from gpjax_amd import linalg
+from oracle import gp_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+EPS = np.finfo(np.float64).eps
+KCLS = {"rbf": gpx.kernels.RBF, "matern12": gpx.kernels.Matern12,
+        "matern32": gpx.kernels.Matern32, "matern52": gpx.kernels.Matern52}
+
+
+def _problem(cuda, n, d, kind, seed):
+    rng = np.random.default_rng(seed)
+    X = rng.uniform(-2, 2, (n, d))
+    y = np.sin(X[:, 0]) + 0.1 * rng.standard_normal(n)
+    ls = np.exp(rng.uniform(np.log(0.5), np.log(2.0), d)) * np.sqrt(d)
+    k = KCLS[kind](lengthscale=ls, variance=1.3)
+    mf = gpx.mean_functions.Constant(gpx.parameters.Real(0.2))
+    post = gpx.gps.Prior(mean_function=mf, kernel=k, jitter=1e-6) * \
+        gpx.likelihoods.Gaussian(num_datapoints=n, obs_stddev=0.3)
+    D = gpx.Dataset(X=torch.tensor(X, device=cuda), y=torch.tensor(y.reshape(-1, 1), device=cuda))
+    return X, y, ls, k, post, D
+
+
+def _grads(post, k):
+    return np.concatenate([k.lengthscale.value.grad.cpu().numpy(),
+                           [k.variance.value.grad.item(),
+                            post.likelihood.obs_stddev.value.grad.item(),
+                            post.prior.mean_function.constant.value.grad.item()]])
+
+
+def _ref_grads(g):
+    return np.concatenate([np.atleast_1d(g["lengthscale"]),
+                           [g["variance"], g["obs_stddev"], g["mean"]]])
+
+
+@pytest.mark.parametrize("n,d,kind", [
+    (1, 1, "rbf"), (127, 16, "matern12"), (128, 16, "matern32"), (128, 17, "matern52"),
+    (3, 2, "matern52"), (129, 5, "rbf"), (385, 3, "matern52")])
+def test_small_mll_routes(cuda, n, d, kind):
+    """The float64 gates of the objective: 1e-10 on the value, 1e-8 on the gradient."""
+    X, y, ls, k, post, D = _problem(cuda, n, d, kind, 7 * n + d)
+    v = gpx.objectives.conjugate_mll(post, D, precision="fp64")
+    v.backward()
+    ref = O.conjugate_mll_grad(kind, X, y, ls, 1.3, 0.3, mean=0.2)
+    g, gr = _grads(post, k), _ref_grads(ref)
+    assert abs(v.item() - ref["mll"]) <= 1e-10 * abs(ref["mll"]) + 1e-12
+    assert np.linalg.norm(g - gr) <= 1e-8 * np.linalg.norm(gr) + 1e-12
+
+
+@pytest.mark.parametrize("n", [2100, 2305])
+def test_loocv_routes(cuda, n):
+    """Either side of the gradient pass's two tile widths, at the float64 gates."""
+    X, y, ls, k, post, D = _problem(cuda, n, 3, "matern32", n)
+    v = gpx.objectives.conjugate_loocv(post, D, precision="fp64")
+    v.backward()
+    ref = O.conjugate_loocv_grad("matern32", X, y, ls, 1.3, 0.3, 1e-6, 0.2)
+    g, gr = _grads(post, k), _ref_grads(ref)
+    assert abs(v.item() - ref["loocv"]) <= 1e-10 * abs(ref["loocv"])
+    assert np.linalg.norm(g - gr) <= 1e-8 * np.linalg.norm(gr)
+
+
+@pytest.mark.parametrize("n", [1, 128, 129, 300, 1153, 4096, 4097])
+def test_inverse_in_the_sweep_against_the_solve(cuda, n):
+    """log N(y; 0, A) through the swept inverse (n <= 4,096) against the factor and the
+    general triangular solve, for A = exp(-|i - j| / 8) + I (condition below 20): both
+    quadratic terms within 8 (n + 1) eps cond of the exact one, the log-determinants
+    within n eps each."""
+    i = torch.arange(n, dtype=torch.float64, device=cuda)
+    A = torch.exp(-(i[:, None] - i[None, :]).abs() / 8) + torch.eye(n, dtype=torch.float64,
+                                                                    device=cuda)
+    y = torch.sin(3.0 * i + 1.0)
+    out = linalg.mvn_log_prob(torch.zeros_like(y), A, y)
+    L, logdet, info = linalg.cholesky_with_info(A)
+    quad = linalg.solve_triangular(L, y[:, None]).square().sum()
+    assert int(info) == 0
+    assert abs(out[2] - quad) <= 2 * 8 * (n + 1) * EPS * 20 * quad
+    assert abs(out[1] - logdet) <= 4 * n * EPS * max(1.0, abs(float(logdet)))
+
+
+@pytest.mark.parametrize("kind", list(KCLS))
+@pytest.mark.parametrize("d", [1, 4, 5, 16, 33])
+def test_builders_at_ragged_sizes(cuda, kind, d):
+    """Entries of the gram and the cross-covariance at sizes around the builder's tiles,
+    to the relative error of the squared distance (d + 4 roundings) times its condition
+    in the exponential (below 40 at these inputs), 1e-13 at least."""
+    rng = np.random.default_rng(d)
+    ls = rng.uniform(0.7, 2.0, d) * np.sqrt(d)
+    k = KCLS[kind](lengthscale=ls, variance=1.7)
+    tol = max(1e-13, 40 * (d + 4) * EPS)
+    for n, m in [(1, 1), (63, 65), (129, 300), (257, 1)]:
+        X, Z = rng.normal(size=(n, d)), rng.normal(size=(m, d))
+        C = k.cross_covariance(torch.tensor(X, device=cuda), torch.tensor(Z, device=cuda))
+        np.testing.assert_allclose(C.cpu().numpy(), O.cross_covariance(kind, X, Z, ls, 1.7),
+                                   rtol=tol, atol=1e-15)
+        G = k.gram(torch.tensor(X, device=cuda)).cpu().numpy()
+        np.testing.assert_allclose(G, O.gram(kind, X, ls, 1.7), rtol=tol, atol=1e-15)
+
+
+@pytest.mark.parametrize("n,m", [(4099, 20), (20011, 257)])
+def test_elbo_odd_widths(cuda, n, m):
+    """The collapsed bound and its gradient at odd widths, at the gates of the float64
+    path: 1e-9 on the value, 1e-7 on the gradient."""
+    rng = np.random.default_rng(n)
+    X = rng.uniform(0, 1, (n, 8))
+    y = np.sin(4 * X[:, 0]) + 0.1 * rng.standard_normal(n)
+    Z = X[rng.permutation(n)[:m]]
+    ls = rng.uniform(0.2, 0.6, 8)
+    k = KCLS["matern32"](lengthscale=ls, variance=1.3)
+    mf = gpx.mean_functions.Constant(gpx.parameters.Real(0.2))
+    post = gpx.gps.Prior(mean_function=mf, kernel=k) * \
+        gpx.likelihoods.Gaussian(num_datapoints=n, obs_stddev=0.3)
+    q = gpx.variational_families.CollapsedVariationalGaussian(
+        posterior=post, inducing_inputs=torch.tensor(Z, device=cuda), jitter=1e-6)
+    D = gpx.Dataset(X=torch.tensor(X, device=cuda), y=torch.tensor(y.reshape(-1, 1), device=cuda))
+    v = gpx.objectives.collapsed_elbo(q, D)
+    v.backward()
+    ref = O.collapsed_elbo_grad("matern32", X, y, Z, ls, 1.3, 0.3, 1e-6, 0.2)
+    g, gr = _grads(post, k), _ref_grads(ref)
+    assert abs(v.item() - ref["elbo"]) <= 1e-9 * abs(ref["elbo"])
+    assert np.linalg.norm(g - gr) <= 1e-7 * np.linalg.norm(gr)
+    gz = q.inducing_inputs.value.grad.cpu().numpy()
+    assert np.abs(gz - ref["Z"]).max() <= 1e-7 * np.abs(ref["Z"]).max()
