@@ -809,8 +809,10 @@ int elbo_forward_impl(int kind, const ElboArith& ea, const double* x, const doub
   double* T = at<double>(ws, Lo.off_T);
   double* Kb = at<double>(ws, Lo.off_K);
   double* Kinv = at<double>(ws, Lo.off_Kinv);
+  // Mixed: G_P is rounded to float32, so its inverses take the fixed order of sums.
+  const int ar = ea.f32 ? AR_F64_SEQ : AR_F64;
   Factor<double> FK{Kb, at<double>(ws, Lo.off_XK), mp, T, at<double>(ws, Lo.off_liK),
-                    at<double>(ws, Lo.off_ldK), at<int>(ws, Lo.off_ifK), AR_F64, AR_F64, s};
+                    at<double>(ws, Lo.off_ldK), at<int>(ws, Lo.off_ifK), ar, ar, s};
   // The Kzz branch (Kzz + jitter I with identity pad, its factor, inverse factor
   // and Kzz^-1 = X^T X, lower tiles then mirrored) needs nothing from the data:
   // it runs on a library stream (aux stream 0, events 6 and 7) while the chunks
@@ -828,8 +830,8 @@ int elbo_forward_impl(int kind, const ElboArith& ea, const double* x, const doub
     FK.s = s2;
     GPK_TRY(launch_kernel_matrix<double>(kind, z, m, z, m, d, theta, nls, jitter, 1, Kb, mp, mp,
                                          mp, true, s2));
-    GPK_TRY(FK.factor(mp, false, true));
-    GPK_TRY(launch_gemm<double, double, double>(AR_F64, true, true, FK.X, mp, FK.X, mp, Kinv, mp,
+    GPK_TRY(ea.f32 ? FK.factor_seq(mp, false) : FK.factor(mp, false, true));
+    GPK_TRY(launch_gemm<double, double, double>(ar, true, true, FK.X, mp, FK.X, mp, Kinv, mp,
                                                 mp, mp, mp, 1.0, false, true, KR_GE_M, s2));
     hipLaunchKernelGGL(mirror_kernel, dim3(cdiv(mp * mp, 256)), dim3(256), 0, s2, Kinv, mp, mp);
     GPK_LAUNCH_CHECK();
@@ -874,15 +876,16 @@ int elbo_forward_impl(int kind, const ElboArith& ea, const double* x, const doub
                      theta, nls);
   GPK_LAUNCH_CHECK();
   Factor<double> FC{Cb, at<double>(ws, Lo.off_XC), mp, T, at<double>(ws, Lo.off_liC),
-                    at<double>(ws, Lo.off_ldC), at<int>(ws, Lo.off_ifC), AR_F64, AR_F64, s};
+                    at<double>(ws, Lo.off_ldC), at<int>(ws, Lo.off_ifC), ar, ar, s};
   // The Kzz branch has joined, so the look-ahead's second stream is free here.
-  GPK_TRY(FC.factor(mp, true, true));
+  GPK_TRY(ea.f32 ? FC.factor_seq(mp, true) : FC.factor(mp, true, true));
   // 3. c = C^-1 b = X_C^T X_C b
   GPK_TRY(launch_trmv<double>(FC.X, mp, mp, b, u, false, vpart, s));
-  GPK_TRY(launch_trmv<double>(FC.X, mp, mp, u, cvec, true, vpart, s));
+  GPK_TRY(launch_trmv<double>(FC.X, mp, mp, u, cvec, true, vpart, s, Batch(), 1, false,
+                              ea.f32 ? 1024 : 0));
   // 4. C^-1 = X^T X (lower tiles, then mirrored; Kzz^-1 came with the Kzz branch)
   double* Cinv = at<double>(ws, Lo.off_Cinv);
-  GPK_TRY(launch_gemm<double, double, double>(AR_F64, true, true, FC.X, mp, FC.X, mp, Cinv, mp,
+  GPK_TRY(launch_gemm<double, double, double>(ar, true, true, FC.X, mp, FC.X, mp, Cinv, mp,
                                               mp, mp, mp, 1.0, false, true, KR_GE_M, s));
   hipLaunchKernelGGL(mirror_kernel, dim3(cdiv(mp * mp, 256)), dim3(256), 0, s, Cinv, mp, mp);
   GPK_LAUNCH_CHECK();

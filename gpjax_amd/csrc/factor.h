@@ -118,14 +118,30 @@ struct Factor {
   int64_t tri_unit = NB;
 
   double* dblk_at(int64_t o) const { return dblk ? dblk + (o / NB) * NB * NB : nullptr; }
+  // Float64 with every sum in the order of its index (ar_potrf = ar_trtri = AR_F64_SEQ,
+  // no batch): the column-sweep leaf, 128-tiles, the recursion or the look-ahead.  For
+  // matrices whose inverse is then rounded to float32 (the mixed collapsed bound's G_P):
+  // a last-bit change of the order moves some of its entries to the other float32
+  // neighbour, and the gradient in Z, a difference of large terms, by 1e-9 to 6e-9.
+  // N = 1e6, M = 2,048: 79.4 ms, against 75.7 on the faster routes.
+  bool seq() const { return ar_potrf == AR_F64_SEQ; }
+  int factor_seq(int64_t n, bool streams) {
+    GPK_TRY(factor_only(n, streams));
+    return trtri(0, n);
+  }
   int leaf(int64_t o) {
+    if constexpr (std::is_same<TS, double>::value) {
+      if (seq())
+        return launch_leaf_sweep(L, X, ld, o, leafinv + (o / NB) * NB * NB, leafld + o / NB,
+                                 leafinfo + o / NB, s);
+    }
     return launch_leaf<TS>(L, X, ld, o, leafinv + (o / NB) * NB * NB, leafld + o / NB,
                            leafinfo + o / NB, dblk_at(o), s, bt);
   }
   // Solve Y L^T = B in place, B = L[row0 : row0+m, o : o+n], triangle L[o:o+n, o:o+n].
   int trsm(int64_t row0, int64_t m, int64_t o, int64_t n) {
     if (n == NB) {
-      if (ar_potrf != AR_F64) {
+      if (ar_potrf != AR_F64 && !seq()) {
         // float32 storage: the leaf also left L11^-1 in float32 in X's diagonal
         // block, so the product takes the Cholesky updates' split arithmetic.
         return launch_gemm<TS, TS, TS>(ar_potrf, false, false, L + row0 * ld + o, ld,
@@ -135,12 +151,12 @@ struct Factor {
       }
       const double* inv = leafinv + (o / NB) * NB * NB;
       if constexpr (std::is_same<TS, double>::value) {
-        if (m / NB * bt.count <= TRSM_STRIP_TILES)
+        if (m / NB * bt.count <= TRSM_STRIP_TILES && !seq())
           return launch_trsm_strip(L + row0 * ld + o, ld, m, inv, s, bt);
       }
       // In place: a workgroup must own its rows' NB columns, so this launch must
       // not take the FP64 products' smaller tiles (it has more tiles than they do).
-      return launch_gemm<TS, double, TS>(AR_F64, false, false, L + row0 * ld + o, ld, inv, NB,
+      return launch_gemm<TS, double, TS>(seq() ? AR_F64_SEQ : AR_F64, false, false, L + row0 * ld + o, ld, inv, NB,
                                          L + row0 * ld + o, ld, m, NB, NB, 1.0, false, false,
                                          KR_FULL, s, nullptr, bt);
     }

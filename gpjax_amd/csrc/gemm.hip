@@ -91,7 +91,7 @@ __device__ __forceinline__ bool gemm_tile(const GemmParams& p, int64_t b, int64_
   return true;
 }
 
-template <int AR, typename TA, typename TB, typename TC, bool A_KM, bool B_KN>
+template <int AR, typename TA, typename TB, typename TC, bool A_KM, bool B_KN, bool SEQ>
 __global__ __launch_bounds__(WaveLayout<AR>::NT) void gemm_kernel(GemmParams p) {
   typedef WaveLayout<AR> WL;
   __shared__ __align__(16) char smem[smem_bytes<AR>()];
@@ -103,7 +103,7 @@ __global__ __launch_bounds__(WaveLayout<AR>::NT) void gemm_kernel(GemmParams p) 
   const int64_t m0 = mt * TILE, n0 = nt * TILE;
   typename AccT<AR>::vec acc[4][WL::NJ];
   if constexpr (AR == AR_F64) {
-    mainloop_f64<TA, TB, A_KM, B_KN>(static_cast<const TA*>(p.A), p.lda,
+    mainloop_f64<TA, TB, A_KM, B_KN, SEQ>(static_cast<const TA*>(p.A), p.lda,
                                      static_cast<const TB*>(p.B), p.ldb, m0, n0, kb, ke, acc,
                                      smem);
   } else {
@@ -346,21 +346,21 @@ __global__ __launch_bounds__(256) void step_solve_kernel(double* B, double* N, i
   else inverse_strip(N, ld, inv, ((int64_t)blockIdx.x - nb) * 16);
 }
 
-template <int AR, typename TA, typename TB, typename TC, bool A_KM, bool B_KN>
+template <int AR, typename TA, typename TB, typename TC, bool A_KM, bool B_KN, bool SEQ>
 int launch_t(const GemmParams& p, hipStream_t s) {
   const dim3 grid((unsigned)tile_count(p), 1, z_count(p));
-  hipLaunchKernelGGL((gemm_kernel<AR, TA, TB, TC, A_KM, B_KN>), grid,
+  hipLaunchKernelGGL((gemm_kernel<AR, TA, TB, TC, A_KM, B_KN, SEQ>), grid,
                      dim3(WaveLayout<AR>::NT), 0, s, p);
   GPK_LAUNCH_CHECK();
   return GPK_OK;
 }
 
-template <int AR, typename TA, typename TB, typename TC>
+template <int AR, typename TA, typename TB, typename TC, bool SEQ = false>
 int dispatch_layout(bool a_km, bool b_kn, const GemmParams& p, hipStream_t s) {
-  if (!a_km && !b_kn) return launch_t<AR, TA, TB, TC, false, false>(p, s);
-  if (!a_km && b_kn) return launch_t<AR, TA, TB, TC, false, true>(p, s);
-  if (a_km && !b_kn) return launch_t<AR, TA, TB, TC, true, false>(p, s);
-  return launch_t<AR, TA, TB, TC, true, true>(p, s);
+  if (!a_km && !b_kn) return launch_t<AR, TA, TB, TC, false, false, SEQ>(p, s);
+  if (!a_km && b_kn) return launch_t<AR, TA, TB, TC, false, true, SEQ>(p, s);
+  if (a_km && !b_kn) return launch_t<AR, TA, TB, TC, true, false, SEQ>(p, s);
+  return launch_t<AR, TA, TB, TC, true, true, SEQ>(p, s);
 }
 
 template <typename TA, typename TB, typename TC>
@@ -379,6 +379,10 @@ int launch_arith(int arith, bool a_km, bool b_kn, const GemmParams& p, hipStream
         return launch_small<2, 2>(a_km, b_kn, p, s);
     }
     return dispatch_layout<AR_F64, TA, TB, TC>(a_km, b_kn, p, s);
+  }
+  if constexpr (std::is_same<TA, double>::value && std::is_same<TB, double>::value &&
+                std::is_same<TC, double>::value) {
+    if (arith == AR_F64_SEQ) return dispatch_layout<AR_F64, TA, TB, TC, true>(a_km, b_kn, p, s);
   }
   if constexpr (std::is_same<TA, float>::value && std::is_same<TB, float>::value) {
     if (arith == AR_BF16X3)

@@ -158,13 +158,14 @@ constexpr size_t smem_bytes() {
 // One 16-deep k-slab of FP64 matrix-core products from LDS operands stored
 // k-major: a[k * ldp + m], b[k * ldp + n]; the wave owns rows wm*64 .. +64 and
 // columns wn*16*NJ .. +16*NJ.  Product kk takes k = kk, 4 + kk, 8 + kk, 12 + kk, as
-// the small-tile kernels do (gemm.hip), so all tile widths give the same bits.
-template <int NJ = 4>
+// the small-tile kernels do (gemm.hip), so all tile widths give the same bits; SEQ:
+// k = 4 kk .. 4 kk + 3 (AR_F64_SEQ).
+template <int NJ = 4, bool SEQ = false>
 __device__ __forceinline__ void mfma_slab_f64(const double* a, const double* b, int ldp,
                                               int lane, int wm, int wn, f64x4 (&acc)[4][NJ]) {
 #pragma unroll
   for (int kk = 0; kk < 4; ++kk) {
-    const int kr = kk + 4 * (lane >> 4);
+    const int kr = SEQ ? 4 * kk + (lane >> 4) : kk + 4 * (lane >> 4);
     double av[4], bv[NJ];
 #pragma unroll
     for (int i = 0; i < 4; ++i) av[i] = a[kr * ldp + wm * 64 + i * 16 + (lane & 15)];
@@ -250,7 +251,7 @@ struct DirectLoop {
 // ---------------------------------------------------------------------------
 // float64 main loop
 // ---------------------------------------------------------------------------
-template <typename TA, typename TB, bool A_KM, bool B_KN>
+template <typename TA, typename TB, bool A_KM, bool B_KN, bool SEQ = false>
 __device__ __forceinline__ void mainloop_f64(const TA* __restrict__ A, int64_t lda,
                                              const TB* __restrict__ B, int64_t ldb, int64_t m0,
                                              int64_t n0, int64_t kb, int64_t ke,
@@ -308,7 +309,7 @@ __device__ __forceinline__ void mainloop_f64(const TA* __restrict__ A, int64_t l
   for (int64_t sl = 0; sl < nslab; ++sl) {
     const int buf = (int)(sl & 1);
     if (sl + 1 < nslab) gload(kb + (sl + 1) * F64_BK);
-    mfma_slab_f64<NJ>(As + buf * F64_BK * F64_LDP, Bs + buf * F64_BK * F64_LDP, F64_LDP, lane,
+    mfma_slab_f64<NJ, SEQ>(As + buf * F64_BK * F64_LDP, Bs + buf * F64_BK * F64_LDP, F64_LDP, lane,
                       wm, wn, acc);
     if (sl + 1 < nslab) sstore(buf ^ 1);
     __syncthreads();

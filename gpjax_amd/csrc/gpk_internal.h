@@ -255,6 +255,9 @@ template <typename TS>
 int launch_leaf(TS* A, TS* X, int64_t ld, int64_t o, double* leafinv, double* logdet, int* info,
                 const double* dsrc, hipStream_t s, const Batch& bt = Batch());
 
+// The float64 leaf with one FMA per entry and column, in order (Factor::seq).
+int launch_leaf_sweep(double* A, double* X, int64_t ld, int64_t o, double* leafinv,
+                      double* logdet, int* info, hipStream_t s);
 // The float64 leaf at o >= NB together with the update C -= P P^T of the `rest` rows
 // and columns beyond it (lower NB-tiles) by the NB columns P before o and, with
 // `inverse`, of the unfinished rows of the inverse by the finished row before o.
@@ -270,7 +273,8 @@ enum KRange { KR_FULL = 0, KR_GE_N = 1, KR_LE_M = 2, KR_GE_M = 3 };
 // Product arithmetic of the tile GEMM.  AR_FP16X3: float32 operands scaled by a
 // power of two (so that every entry sits well inside the fp16 range), split
 // into fp16 hi + lo planes, products hi*hi + hi*lo + lo*hi.
-enum Arith { AR_F64 = 0, AR_BF16X3 = 3, AR_FP16X3 = 4, AR_BF16X6 = 6 };
+// AR_F64_SEQ: float64 on 128-tiles alone, four consecutive k per product (Factor::seq).
+enum Arith { AR_F64 = 0, AR_F64_SEQ = 1, AR_BF16X3 = 3, AR_FP16X3 = 4, AR_BF16X6 = 6 };
 
 // Tile rule of the FP64 products (double operands, no diagonal side buffer), by the
 // number of 128-tiles of the launch (every tile width sums k in the same order, so
@@ -402,11 +406,12 @@ inline int64_t colreduce_chunks(int64_t rows) {
 // y = X r (trans = false) or y = X^T r (trans = true; add: y += X^T r), X lower
 // triangular np x np (only k <= i is read); float64 accumulation through `partial`
 // (nv x trmv_max_chunks(np) x np doubles).  nv = 1 or 3 right-hand sides, stored
-// np apart in r and in y, share each pass over X.
+// np apart in r and in y, share each pass over X.  rows: the transposed form's row
+// chunk (at least trmv_t_rows, at most 1,024), 0 for the rule above.
 template <typename TS>
 int launch_trmv(const TS* X, int64_t ld, int64_t np, const double* r, double* y, bool trans,
                 double* partial, hipStream_t s, const Batch& bt = Batch(), int nv = 1,
-                bool add = false);
+                bool add = false, int64_t rows = 0);
 
 // Columns per chunk of the recomputed Sigma product below: the widest power of two
 // (64 .. 1,024) whose grid, ceil(np / 256) row blocks x chunks x members, has at

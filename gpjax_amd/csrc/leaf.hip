@@ -380,6 +380,140 @@ __global__ __launch_bounds__(LEAF_THREADS) void leaf_update_kernel(
       C[(mw + lr + 4 * r) * ld + nw + 16 * j + lc] = cv[j][r] - acc[0][j][r];
 }
 
+// The leaf as a right-looking sweep by columns, for Factor::seq: thread t of 1,024 holds
+// the 4 x 4 block at rows 4 (t % 32), columns 4 (t / 32) of one array with the trailing
+// matrix / L below the diagonal and the numerators of X = L^-1, transposed, above it.
+// The half-wave that owns a panel of four columns factors it among its own lanes and
+// publishes it; after one barrier every thread to the right applies the rank-4 update.
+// 67 us, bound by its 32 dependent panels (leaf_kernel: 26.5), but each entry takes one
+// FMA per column, in order.
+constexpr int SWEEP_THREADS = 1024;
+constexpr int EB = 4;
+constexpr int BPR = NB / EB;
+__global__ __launch_bounds__(SWEEP_THREADS) void leaf_sweep_kernel(
+    double* A, double* X, int64_t ld, int64_t o, double* __restrict__ leafinv,
+    double* __restrict__ logdet, int* __restrict__ info) {
+  // pub[buf][kk][i]: the step factors of the four columns of the last panel
+  // (row factor of row i; for rows below the step's column also its column
+  // factor).  Double-buffered across panels.
+  __shared__ double pub[2][EB][NB];
+  __shared__ double dk_s[NB];
+  __shared__ double dinv_s[NB];
+  __shared__ int bad_s;
+  __shared__ double tr_s[NB][NB + 1];
+
+  const int t = threadIdx.x;
+  const int rb = (t % BPR) * EB;   // first row of this thread's block
+  const int cb = (t / BPR) * EB;   // first column (the half-wave t / 32 owns columns cb .. cb+3)
+  const int hl = t % BPR;          // lane within the half-wave: rows 4 hl .. 4 hl + 3
+  const int hbase = (t & 63) & ~(BPR - 1);  // first wave lane of this half-wave
+  // Stage the block through LDS so that global reads stay row-contiguous.
+  for (int e = t; e < NB * NB; e += SWEEP_THREADS) {
+    const int i = e / NB, j = e % NB;
+    tr_s[i][j] = A[(o + i) * ld + o + j];
+  }
+  if (t == 0) bad_s = NB;
+  __syncthreads();
+  double s[EB][EB];
+#pragma unroll
+  for (int a = 0; a < EB; ++a)
+#pragma unroll
+    for (int b = 0; b < EB; ++b) s[a][b] = (cb + b <= rb + a) ? tr_s[rb + a][cb + b] : 0.0;
+
+  for (int p = 0; p < NB / EB; ++p) {
+    const int c0 = p * EB;  // the panel's columns c0 .. c0 + 3
+    if (cb == c0) {
+      // Factor the panel inside this half-wave.  Step k = c0 + kk: the pivot
+      // and the panel's own entries of column k (rows c0 .. c0+3) sit in the
+      // half-wave lane p; each is broadcast from there.  As in the unblocked
+      // sweep, entry (i, j), j > k, takes one FMA with row factor
+      // f_i = s_ik / d_k (1 / d_k on the diagonal) and column factor s_jk / d_k
+      // when i >= j (trailing update of L) or i <= k (numerator of X[j][i]).
+#pragma unroll
+      for (int kk = 0; kk < EB; ++kk) {
+        const int k = c0 + kk;
+        double cv[EB];
+#pragma unroll
+        for (int a = 0; a < EB; ++a) cv[a] = __shfl(s[a][kk], hbase + p);
+        const double piv = cv[kk];
+        const double dk = sqrt(piv);
+        const double inv = 1.0 / dk;
+        double f[EB];
+#pragma unroll
+        for (int a = 0; a < EB; ++a) f[a] = (rb + a == k) ? inv : s[a][kk] * inv;
+#pragma unroll
+        for (int b = kk + 1; b < EB; ++b) {
+          const double g = cv[b] * inv;  // column factor of column c0 + b
+#pragma unroll
+          for (int a = 0; a < EB; ++a) {
+            const int i = rb + a, j = c0 + b;
+            const double fa = (i >= j || i <= k) ? f[a] : 0.0;
+            s[a][b] = fma(-fa, g, s[a][b]);
+          }
+        }
+#pragma unroll
+        for (int a = 0; a < EB; ++a) s[a][kk] = (rb + a == k) ? dk : f[a];
+#pragma unroll
+        for (int a = 0; a < EB; ++a) pub[p & 1][kk][rb + a] = f[a];
+        if (hl == p) {
+          dk_s[k] = dk;
+          dinv_s[k] = inv;
+          if (!(piv > 0.0) && k < bad_s) bad_s = k;
+        }
+      }
+    }
+    __syncthreads();
+    if (cb > c0) {
+      // Rank-4 update of the columns right of the panel, steps in order.
+      const double* P = &pub[p & 1][0][0];
+#pragma unroll
+      for (int kk = 0; kk < EB; ++kk) {
+        const int k = c0 + kk;
+        double fr[EB], g[EB];
+#pragma unroll
+        for (int a = 0; a < EB; ++a) fr[a] = P[kk * NB + rb + a];
+#pragma unroll
+        for (int b = 0; b < EB; ++b) g[b] = P[kk * NB + cb + b];
+#pragma unroll
+        for (int a = 0; a < EB; ++a) {
+          const int i = rb + a;
+          // j = cb + b > k always here; the mask is i >= j or i <= k
+          const double flo = fr[a];
+          const double fhi = (i <= k) ? fr[a] : 0.0;
+#pragma unroll
+          for (int b = 0; b < EB; ++b) {
+            const double fa = (i >= cb + b) ? flo : fhi;
+            s[a][b] = fma(-fa, g[b], s[a][b]);
+          }
+        }
+      }
+    }
+  }
+
+  // L (lower incl. diagonal) and X (from the upper part, transposed) staged
+  // in LDS for row-contiguous writes.
+  __syncthreads();
+#pragma unroll
+  for (int a = 0; a < EB; ++a)
+#pragma unroll
+    for (int b = 0; b < EB; ++b) tr_s[rb + a][cb + b] = s[a][b];
+  if (t < NB) dk_s[t] = log(dk_s[t]);
+  __syncthreads();
+  for (int e = t; e < NB * NB; e += SWEEP_THREADS) {
+    const int i = e / NB, j = e % NB;
+    A[(o + i) * ld + o + j] = (j <= i) ? tr_s[i][j] : 0.0;
+    const double v = (j < i) ? tr_s[j][i] : (j == i ? dinv_s[i] : 0.0);
+    X[(o + i) * ld + o + j] = v;
+    leafinv[e] = v;
+  }
+  if (t == 0) {
+    double ld_acc = 0.0;  // in column order, as the sweep produced the pivots
+    for (int k = 0; k < NB; ++k) ld_acc += dk_s[k];
+    *logdet = 2.0 * ld_acc;
+    *info = bad_s < NB ? (int)(o + bad_s + 1) : 0;
+  }
+}
+
 }  // namespace
 
 template <typename TS>
@@ -387,6 +521,14 @@ int launch_leaf(TS* A, TS* X, int64_t ld, int64_t o, double* leafinv, double* lo
                 const double* dsrc, hipStream_t s, const Batch& bt) {
   hipLaunchKernelGGL(leaf_kernel<TS>, dim3(1, 1, bt.count), dim3(LEAF_THREADS), 0, s, A, X, ld,
                      o, leafinv, logdet, info, dsrc, bt);
+  GPK_LAUNCH_CHECK();
+  return GPK_OK;
+}
+
+int launch_leaf_sweep(double* A, double* X, int64_t ld, int64_t o, double* leafinv,
+                      double* logdet, int* info, hipStream_t s) {
+  hipLaunchKernelGGL(leaf_sweep_kernel, dim3(1), dim3(SWEEP_THREADS), 0, s, A, X, ld, o, leafinv,
+                     logdet, info);
   GPK_LAUNCH_CHECK();
   return GPK_OK;
 }

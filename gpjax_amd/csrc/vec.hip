@@ -470,7 +470,8 @@ __global__ void mfma_selftest_kernel(double* out64, float* outbf) {
 
 template <typename TS>
 int launch_trmv(const TS* X, int64_t ld, int64_t np, const double* r, double* y, bool trans,
-                double* partial, hipStream_t s, const Batch& bt, int nv, bool add) {
+                double* partial, hipStream_t s, const Batch& bt, int nv, bool add,
+                int64_t rows) {
   if (np % NB) {
     set_error("trmv: size %lld not a multiple of %d", (long long)np, NB);
     return GPK_ERR_BAD_ARG;
@@ -497,7 +498,7 @@ int launch_trmv(const TS* X, int64_t ld, int64_t np, const double* r, double* y,
     if (nc > 1)
       hipLaunchKernelGGL(trmv_n_reduce, gvec, dim3(256), 0, s, partial, np, nc, nv, y, bt);
   } else {
-    const int64_t rc = trmv_t_rows(np, bt.count);
+    const int64_t rc = rows ? rows : trmv_t_rows(np, bt.count);
     const int64_t nc = (np + rc - 1) / rc;
     const dim3 grid((unsigned)(np / TRMV_TC), (unsigned)nc, bt.count);
     if (nv == 1)
@@ -515,9 +516,9 @@ int launch_trmv(const TS* X, int64_t ld, int64_t np, const double* r, double* y,
 }
 
 template int launch_trmv<double>(const double*, int64_t, int64_t, const double*, double*, bool,
-                                 double*, hipStream_t, const Batch&, int, bool);
+                                 double*, hipStream_t, const Batch&, int, bool, int64_t);
 template int launch_trmv<float>(const float*, int64_t, int64_t, const double*, double*, bool,
-                                double*, hipStream_t, const Batch&, int, bool);
+                                double*, hipStream_t, const Batch&, int, bool, int64_t);
 
 int launch_sigma_matvec(int kind, const double* x, int64_t n, int64_t np, int d,
                         const double* theta, int nls, double jitter, const double* a, double* v,

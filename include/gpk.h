@@ -17,8 +17,8 @@
  *     through `prec`.
  *   - Some calls fork work onto those library streams and join it back into
  *     `stream` with events before they return (the look-ahead Cholesky for
- *     n > 4,096 in float64 and n > 1,920 in the mixed precisions, also for the
- *     collapsed ELBO's M x M factor when m > 4,096, the batched size buckets, the collapsed ELBO's Kzz-side work during its
+ *     n, or the collapsed ELBO's m, > 4,096 in float64 and > 1,920 in the mixed
+ *     precisions, the batched size buckets, the collapsed ELBO's Kzz-side work during its
  *     streamed chunks): to the caller the call stays
  *     ordered on `stream`, and under HIP-graph capture the fork and join become
  *     graph edges.  The streams and events are created by a thread's first
