@@ -308,12 +308,14 @@ __global__ __launch_bounds__(WaveLayout<AR>::NT) void adjoint_kernel(int kind,
 
 // The FP64 pass on 64 x 64 tiles (inputs of up to ADJ_DCH dimensions), for problems
 // whose 128-tiles leave most of the chip idle: four independent waves of 32 x 32, each
-// reading its operands straight from global memory (DirectLoop).  Tiles (I, J),
+// reading its operands straight from global memory (DirectLoop), down the columns of X:
+// a column read takes whole 128-byte lines, where rows of X^T would touch 16 lines per
+// instruction (158 us at np = 2,048, and the transpose before it).  Tiles (I, J),
 // I >= J, of 64 rows; each writes its own partial sums.  k runs from the row tile at
 // the granularity of KG, in the large tiles' order.  np = 2,048: 285 us on 136 large
-// tiles, 158 us.
+// tiles, 115 us.
 constexpr int AT = 64;
-template <int DMAX, bool XT>
+template <int DMAX>
 __global__ __launch_bounds__(256, 2) void adjoint_small_kernel(
     int kind, const double* __restrict__ X, int64_t ld, int64_t np, const double* __restrict__ x,
     int64_t n, int d, const double* __restrict__ theta, int nls, const double* __restrict__ alpha,
@@ -332,7 +334,7 @@ __global__ __launch_bounds__(256, 2) void adjoint_small_kernel(
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   const int64_t mw = m0 + (w >> 1) * 32, nw = n0 + (w & 1) * 32;
   f64x4 acc[2][2];
-  DirectLoop<!XT, !XT, 2, 2> loop(X, ld, X, ld, mw, nw, lane, dense ? 0 : m0 / KG * KG, np);
+  DirectLoop<true, true, 2, 2> loop(X, ld, X, ld, mw, nw, lane, dense ? 0 : m0 / KG * KG, np);
   for (int e = t; e < AT * DMAX; e += 256) {
     const int r = e / DMAX, q = e % DMAX;
     if (q < d) {
@@ -419,18 +421,12 @@ __global__ __launch_bounds__(256, 2) void adjoint_small_kernel(
 int launch_small_adjoint(int kind, const double* X, int64_t ld, int64_t np, const double* x,
                          int64_t n, int d, const double* theta, int nls, const double* alpha,
                          double* partial, hipStream_t s, const Batch& bt, const double* beta,
-                         bool dense, bool xt) {
+                         bool dense) {
   const int64_t nt = np / AT;
   const dim3 grid((unsigned)(nt * (nt + 1) / 2), 1, bt.count);
-#define GPK_ADJS(DM)                                                                          \
-  do {                                                                                        \
-    if (xt)                                                                                   \
-      hipLaunchKernelGGL((adjoint_small_kernel<DM, true>), grid, dim3(256), 0, s, kind, X, ld, \
-                         np, x, n, d, theta, nls, alpha, beta, dense ? 1 : 0, partial, bt);   \
-    else                                                                                      \
-      hipLaunchKernelGGL((adjoint_small_kernel<DM, false>), grid, dim3(256), 0, s, kind, X,   \
-                         ld, np, x, n, d, theta, nls, alpha, beta, dense ? 1 : 0, partial, bt); \
-  } while (0)
+#define GPK_ADJS(DM)                                                                        \
+  hipLaunchKernelGGL(adjoint_small_kernel<DM>, grid, dim3(256), 0, s, kind, X, ld, np, x, n, \
+                     d, theta, nls, alpha, beta, dense ? 1 : 0, partial, bt)
   if (d <= 1) GPK_ADJS(1);
   else if (d <= 2) GPK_ADJS(2);
   else if (d <= 4) GPK_ADJS(4);
@@ -488,9 +484,14 @@ int launch_adjoint(int kind, int arith, const TS* X, int64_t ld, int64_t np, con
     return GPK_ERR_BAD_ARG;
   }
   if constexpr (std::is_same<TS, double>::value) {
-    if (arith == AR_F64 && adjoint_small(np, d, bt.count))
+    if (arith == AR_F64 && adjoint_small(np, d)) {
+      if (xt) {
+        set_error("adjoint: the 64-wide pass reads X, not its transpose");
+        return GPK_ERR_BAD_ARG;
+      }
       return launch_small_adjoint(kind, X, ld, np, x, n, d, theta, nls, alpha, partial, s, bt,
-                                  beta, dense, xt);
+                                  beta, dense);
+    }
   }
   if (arith == AR_F64)
     return launch_ar<AR_F64, TS>(kind, X, ld, np, x, n, d, theta, nls, alpha, partial, s, bt,

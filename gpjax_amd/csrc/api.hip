@@ -171,7 +171,7 @@ Layout make_layout(int64_t n, int64_t d, int prec, int spk = -1) {
   L.off_part = o; o += al((size_t)L.nvec * nchunk * np * sizeof(double));
   L.off_skip = o; o += al(sizeof(int));
   L.off_gpart = o;
-  o += al((size_t)adjoint_tiles(prec == GPK_PREC_FP64, np, (int)d, 1) * (d + 2) * sizeof(double));
+  o += al((size_t)adjoint_tiles(prec == GPK_PREC_FP64, np, (int)d) * (d + 2) * sizeof(double));
   L.off_scal = o; o += al(16 * sizeof(double));
   L.off_probe = o; o += al(3 * NPROBE * sizeof(double));
   L.total = o;
@@ -613,7 +613,7 @@ struct Variant {
 // touches 16 lines per instruction (n = 2,000: 158 -> 115 us and no transpose).
 Variant single_variant(bool f64, int64_t np, int d) {
   Variant v;
-  v.adj_transposed = !(f64 && adjoint_small(np, d, 1));
+  v.adj_transposed = !(f64 && adjoint_small(np, d));
   return v;
 }
 
@@ -765,7 +765,8 @@ int mll_backward_t(int kind, const Arith3& ar, const double* x, int64_t n, int d
                    const Variant* variant = nullptr) {
   const int64_t np = Lo.np;
   const bool f64 = std::is_same<TS, double>::value;
-  const Variant vr = variant ? *variant : single_variant(f64, np, d);
+  Variant vr = variant ? *variant : single_variant(f64, np, d);
+  if (f64 && adjoint_small(np, d)) vr.adj_transposed = false;
   double* gpart = at<double>(ws, Lo.off_gpart);
   const float* fs = f64 ? nullptr : at<float>(ws, Lo.off_scal) + 2;
   if (vr.adj_transposed) {
@@ -785,8 +786,8 @@ int mll_backward_t(int kind, const Arith3& ar, const double* x, int64_t n, int d
                                bt, nullptr, false, fs));
   }
   hipLaunchKernelGGL(finalize_bwd_kernel, dim3((unsigned)(nls + 3), 1, bt.count), dim3(256), 0, s,
-                     gpart, adjoint_tiles(f64, np, d, bt.count), nls, theta, at<double>(ws, Lo.off_alpha), n,
-                     gbar, grad, bt);
+                     gpart, adjoint_tiles(f64, np, d), nls, theta, at<double>(ws, Lo.off_alpha),
+                     n, gbar, grad, bt);
   GPK_LAUNCH_CHECK();
   return GPK_OK;
 }
@@ -1067,7 +1068,7 @@ int loocv_backward_t(int kind, const Arith3& ar3, const double* x, int64_t n, in
                              at<double>(ws, Lo.off_alpha), gpart, s, Batch(), w, true, nullptr,
                              vr.adj_transposed));
   hipLaunchKernelGGL(finalize_bwd_kernel, dim3((unsigned)(nls + 3)), dim3(256), 0, s, gpart,
-                     adjoint_tiles(f64, np, d, 1), nls, theta, w, n, gbar, grad, Batch());
+                     adjoint_tiles(f64, np, d), nls, theta, w, n, gbar, grad, Batch());
   GPK_LAUNCH_CHECK();
   return GPK_OK;
 }

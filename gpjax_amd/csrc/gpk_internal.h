@@ -346,18 +346,22 @@ int launch_tri_level(int arith, const TriLevel& lev, int64_t max_m, int64_t max_
 int launch_trsm_strip(double* B, int64_t ld, int64_t m, const double* inv, hipStream_t s,
                       const Batch& bt = Batch());
 
-// True when the FP64 pass below runs on 64-tiles, and the number of partial records a
-// call writes (each nls + 2 doubles): one per tile.  Up to 600 128-tiles, about
-// where those fill the chip's two workgroups per CU: MLL + gradient at n = 2,000 1.60
-// -> 1.47 ms and n = 4,000 even, but n = 6,000 (1,128 tiles) 8.5 -> 8.9 ms and a batch
-// of 4,096 small GPs 60.8 -> 62.6 ms with the small tiles.
+// True when the FP64 pass below runs on 64-tiles (which read X down its columns, never
+// its transpose), and the number of partial records a call writes (each nls + 2
+// doubles): one per tile.  Up to 600 128-tiles, about where those fill the chip's two
+// workgroups per CU: MLL + gradient at n = 2,000 1.60 -> 1.47 ms and n = 4,000 even, but
+// n = 6,000 (1,128 tiles) 8.5 -> 8.9 ms with the small tiles.  By np and d alone: the
+// width is part of the order of the sums, and a batch member's must not depend on how
+// many members share a launch.  Batches, 128-wide / 64-wide (MLL + gradient): 8 GPs of
+// 1,024 rows 1.15 / 1.00 ms, 400 of 512 3.36 / 3.19 ms, 50 of 2,048 11.94 / 11.86 ms,
+// 400 of 1,024 15.5 / 15.8 ms (d = 8: 18.3 / 16.9), 4,096 of 32 to 1,024 57.5 / 58.7 ms.
 constexpr int64_t ADJ_SMALL_TILES = 600;
-inline bool adjoint_small(int64_t np, int d, int64_t members) {
+inline bool adjoint_small(int64_t np, int d) {
   const int64_t T = np / NB;
-  return d <= 32 && T * (T + 1) / 2 * members <= ADJ_SMALL_TILES;
+  return d <= 32 && T * (T + 1) / 2 <= ADJ_SMALL_TILES;
 }
-inline int64_t adjoint_tiles(bool f64, int64_t np, int d, int64_t members) {
-  const int64_t T = f64 && adjoint_small(np, d, members) ? np / 64 : np / NB;
+inline int64_t adjoint_tiles(bool f64, int64_t np, int d) {
+  const int64_t T = f64 && adjoint_small(np, d) ? np / 64 : np / NB;
   return T * (T + 1) / 2;
 }
 
@@ -374,7 +378,8 @@ int launch_adjoint(int kind, int arith, const TS* X, int64_t ld, int64_t np, con
                    double* partial, hipStream_t s, const Batch& bt = Batch(),
                    const double* beta = nullptr, bool dense = false,
                    const float* fscale = nullptr, bool xt = false);
-// xt: the operand passed is U = X^T (upper, row-major) from launch_lower_to_upper.
+// xt: the operand passed is U = X^T (upper, row-major) from launch_lower_to_upper
+// (refused where adjoint_small).
 
 // U = X^T for lower-triangular X (np x np, np a multiple of NB): upper U with
 // zeros below the diagonal inside its diagonal NB-tiles.
@@ -383,16 +388,18 @@ int launch_lower_to_upper(const TS* X, TS* U, int64_t ld, int64_t np, hipStream_
                           const Batch& bt = Batch());
 
 // Row chunk of launch_trmv's transposed form over its 64-column blocks: the widest of
-// 1,024 .. 128 rows whose grid (column blocks x chunks x members) has at least 1,024
-// workgroups, 128 if none has; and the most chunks it makes of np rows.
-inline int64_t trmv_t_rows(int64_t np, int64_t members) {
+// 1,024 .. 128 rows whose grid (column blocks x chunks) has at least 1,024 workgroups,
+// 128 if none has; and the chunks it makes of np rows.  By np alone (as the two rules
+// below and colreduce_rows): the members of a batch add to the grid, but a member's sums
+// must not depend on how many others are computed with it.
+inline int64_t trmv_t_rows(int64_t np) {
   const int64_t blocks = (np + 63) / 64;
   int64_t rc = 1024;
-  while (rc > 128 && blocks * ((np + rc - 1) / rc) * members < 1024) rc /= 2;
+  while (rc > 128 && blocks * ((np + rc - 1) / rc) < 1024) rc /= 2;
   return rc;
 }
 inline int64_t trmv_max_chunks(int64_t np) {
-  const int64_t rc = trmv_t_rows(np, 1);
+  const int64_t rc = trmv_t_rows(np);
   return (np + rc - 1) / rc;
 }
 // Row chunk of launch_colreduce, by the number of rows alone: a column's sum does not
@@ -414,17 +421,16 @@ int launch_trmv(const TS* X, int64_t ld, int64_t np, const double* r, double* y,
                 bool add = false, int64_t rows = 0);
 
 // Columns per chunk of the recomputed Sigma product below: the widest power of two
-// (64 .. 1,024) whose grid, ceil(np / 256) row blocks x chunks x members, has at
-// least 1,024 workgroups (four waves per SIMD), 64 if none has.
-inline int64_t sigma_mv_chunk(int64_t np, int64_t members) {
+// (64 .. 1,024) whose grid, ceil(np / 256) row blocks x chunks, has at least 1,024
+// workgroups (four waves per SIMD), 64 if none has.
+inline int64_t sigma_mv_chunk(int64_t np) {
   const int64_t rows = (np + 255) / 256;
   int64_t cw = 1024;
-  while (cw > 64 && rows * ((np + cw - 1) / cw) * members < 1024) cw /= 2;
+  while (cw > 64 && rows * ((np + cw - 1) / cw) < 1024) cw /= 2;
   return cw;
 }
-// Most chunks any member count gives (the partial sums' room).
 inline int64_t sigma_mv_max_chunks(int64_t np) {
-  const int64_t cw = sigma_mv_chunk(np, 1);
+  const int64_t cw = sigma_mv_chunk(np);
   return (np + cw - 1) / cw;
 }
 

@@ -498,7 +498,7 @@ int launch_trmv(const TS* X, int64_t ld, int64_t np, const double* r, double* y,
     if (nc > 1)
       hipLaunchKernelGGL(trmv_n_reduce, gvec, dim3(256), 0, s, partial, np, nc, nv, y, bt);
   } else {
-    const int64_t rc = rows ? rows : trmv_t_rows(np, bt.count);
+    const int64_t rc = rows ? rows : trmv_t_rows(np);
     const int64_t nc = (np + rc - 1) / rc;
     const dim3 grid((unsigned)(np / TRMV_TC), (unsigned)nc, bt.count);
     if (nv == 1)
@@ -532,7 +532,7 @@ int launch_sigma_matvec(int kind, const double* x, int64_t n, int64_t np, int d,
     set_error("sigma matvec: %d right-hand sides (1 or 3 supported)", nv);
     return GPK_ERR_BAD_ARG;
   }
-  const int64_t cw = sigma_mv_chunk(np, bt.count);
+  const int64_t cw = sigma_mv_chunk(np);
   const int64_t nc = (np + cw - 1) / cw;
   dim3 grid((unsigned)((np + 255) / 256), (unsigned)nc, bt.count);
 #define GPK_SMV(DM)                                                                           \

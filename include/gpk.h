@@ -318,7 +318,9 @@ int gpk_loocv_backward(int kind, int prec, const double* x, int64_t n, int64_t d
  *   x [offsets[count], d] and y [offsets[count]] (device).
  * theta: device [count][nls + 3], each row in gpk_mll_forward's layout.
  * Problems are grouped by padded size; one group runs as one set of launches
- * with one problem per blockIdx.z.
+ * with one problem per blockIdx.z.  A problem's result and gradient are the same
+ * bits whatever other problems the batch holds, as long as its group runs the same
+ * launch variant (gpk_batched_tune keeps them per padded size and members).
  */
 size_t gpk_batched_workspace_bytes(const int64_t* offsets_host, int64_t count, int64_t d,
                                    int prec);
