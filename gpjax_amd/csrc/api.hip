@@ -602,18 +602,22 @@ int check_ws(const char* fn, const void* ws, size_t have, size_t need) {
 //   evaluating the kernel again;
 // adj_transposed: the fused Sigma^-1 pass reads U = X^T along k (one transpose
 //   first) instead of X down its columns.
-// The single-problem path runs the defaults (single_variant); the batched path takes
-// them per size group from the autotuner's table.
+// The single-problem path runs the defaults; the batched path takes them per size group
+// from the autotuner's table.  Both as far as the size leaves the choice (variant_for).
 struct Variant {
   bool stored_sigma = true;
   bool adj_transposed = true;
 };
-// A single problem's: the FP64 pass on small tiles reads its operands straight into
-// the matrix cores, where a column read takes whole 128-byte lines and a row read
-// touches 16 lines per instruction (n = 2,000: 158 -> 115 us and no transpose).
-Variant single_variant(bool f64, int64_t np, int d) {
-  Variant v;
-  v.adj_transposed = !(f64 && adjoint_small(np, d));
+
+// float64 problems whose solve is one launch (small_solve_kernel).
+bool one_launch_solve(bool f64, int64_t np, int d) { return f64 && np == NB && d <= SOLVE_D; }
+
+// The variant that runs at this size: the one-launch solve evaluates Sigma itself, so a
+// stored copy would be written and not read, and the 64-wide gradient pass reads X down
+// its columns.
+Variant variant_for(Variant v, bool f64, int64_t np, int d) {
+  if (one_launch_solve(f64, np, d)) v.stored_sigma = false;
+  if (f64 && adjoint_small(np, d)) v.adj_transposed = false;
   return v;
 }
 
@@ -621,8 +625,9 @@ template <typename TS>
 int mll_forward_t(int kind, const Arith3& ar, const double* x, const double* y, int64_t n, int d,
                   const double* theta, int nls, double jitter, int iters, void* ws,
                   const Layout& Lo, double* result, hipStream_t s,
-                  const Batch& bt = Batch(), const Variant& vr = Variant()) {
+                  const Batch& bt = Batch(), const Variant& variant = Variant()) {
   const int64_t np = Lo.np;
+  const Variant vr = variant_for(variant, std::is_same<TS, double>::value, np, d);
   const dim3 gv(nblk(np), 1, bt.count);
   TS* L = at<TS>(ws, Lo.off_L);
   TS* X = at<TS>(ws, Lo.off_X);
@@ -667,7 +672,7 @@ int mll_forward_t(int kind, const Arith3& ar, const double* x, const double* y, 
     F.fscale = fs;
   }
 
-  const bool small = f64 && np == NB && d <= SOLVE_D;  // one launch for all of the solve
+  const bool small = one_launch_solve(f64, np, d);
   int* skip = at<int>(ws, Lo.off_skip);
   if (!small) {
     hipLaunchKernelGGL(prep_r_kernel, gv, dim3(256), 0, s, y, theta, nls, n, np, r, skip, bt);
@@ -762,11 +767,10 @@ template <typename TS>
 int mll_backward_t(int kind, const Arith3& ar, const double* x, int64_t n, int d,
                    const double* theta, int nls, double gbar, void* ws, const Layout& Lo,
                    double* grad, hipStream_t s, const Batch& bt = Batch(),
-                   const Variant* variant = nullptr) {
+                   const Variant& variant = Variant()) {
   const int64_t np = Lo.np;
   const bool f64 = std::is_same<TS, double>::value;
-  Variant vr = variant ? *variant : single_variant(f64, np, d);
-  if (f64 && adjoint_small(np, d)) vr.adj_transposed = false;
+  const Variant vr = variant_for(variant, f64, np, d);
   double* gpart = at<double>(ws, Lo.off_gpart);
   const float* fs = f64 ? nullptr : at<float>(ws, Lo.off_scal) + 2;
   if (vr.adj_transposed) {
@@ -981,7 +985,7 @@ __global__ __launch_bounds__(256) void loo_fwd_kernel(const double* __restrict__
 // Y <- diag(c) S, or its transpose S diag(c) (tr), with S symmetric held in its lower
 // 64-tiles (upper tiles are overwritten).  The transpose lets the pass over Y^T Y
 // read both operands along rows (n = 9,000 float64 34.7 -> 33.5 ms, n = 16,000 mixed
-// 63.2 -> 62.4); its small tiles prefer columns (single_variant).  One workgroup per
+// 63.2 -> 62.4); its small tiles prefer columns (variant_for).  One workgroup per
 // lower tile (I, J): it reads only tile (I, J) and writes tiles (I, J) and (J, I), so
 // the update in place has no race.
 constexpr int MT = 64;
@@ -1059,7 +1063,7 @@ int loocv_backward_t(int kind, const Arith3& ar3, const double* x, int64_t n, in
   GPK_TRY(launch_gemm<TS, TS, TS>(ar, true, true, X, np, X, np, Y, np, np, np, np, 1.0, false,
                                   true, KR_GE_M, s));
   const int64_t mt = np / MT;
-  const Variant vr = single_variant(f64, np, d);
+  const Variant vr = variant_for(Variant(), f64, np, d);
   hipLaunchKernelGGL(loo_scale_mirror_kernel<TS>, dim3((unsigned)(mt * (mt + 1) / 2)), dim3(256),
                      0, s, Y, np, at<double>(ws, P.off_c), vr.adj_transposed ? 1 : 0);
   GPK_LAUNCH_CHECK();
@@ -1180,7 +1184,8 @@ uint64_t hash_offsets(const int64_t* off, int64_t count) {
 constexpr int BATCH_STREAMS = GPK_BATCH_STREAMS;
 
 // ---- autotuning of the batched path ----
-// gpk_batched_tune times the launch variants (Variant: 4 combinations) of each
+// gpk_batched_tune times the launch variants (Variant: 4 combinations, fewer where
+// variant_for makes them one) of each
 // size group on the caller's own problems and keeps the fastest in a
 // process-wide table keyed by (device architecture, kernel kind, prec, padded
 // size, member-count class = ceil(log2 members), d), guarded by a mutex;
@@ -1205,6 +1210,7 @@ Variant variant_of(int id) {
   v.adj_transposed = (id & 2) != 0;
   return v;
 }
+int variant_id(const Variant& v) { return (v.stored_sigma ? 1 : 0) | (v.adj_transposed ? 2 : 0); }
 
 // gcnArchName of the current device (cached per device ordinal).
 int current_arch(std::string* arch) {
@@ -1261,7 +1267,7 @@ int run_group(int kind, const Arith3& ar, const double* x, const double* y, int 
   // n is taken per member inside the kernels; np fixes the shapes.
   GPK_TRY(mll_forward_t<TS>(kind, ar, x, y, g.np, d, theta, nls, jitter, iters, wsg, g.lo,
                             result, s, bt, vr));
-  return mll_backward_t<TS>(kind, ar, x, g.np, d, theta, nls, 1.0, wsg, g.lo, grad, s, bt, &vr);
+  return mll_backward_t<TS>(kind, ar, x, g.np, d, theta, nls, 1.0, wsg, g.lo, grad, s, bt, vr);
 }
 
 template <typename TS>
@@ -1355,7 +1361,8 @@ int batched_mll_grad(int kind, int prec, const Arith3& ar, const double* x, cons
 }
 
 // Times every variant of every group (one untimed run, then the mean of
-// `reps` runs between two events on the stream) and records the fastest.
+// `reps` runs between two events on the stream) and records the fastest; variants
+// that are one at the group's size (variant_for) are timed once.
 template <typename TS>
 int batched_tune(int kind, int prec, const Arith3& ar, const double* x, const double* y,
                  const int64_t* off, int64_t count, int d, const double* theta, int nls,
@@ -1380,6 +1387,11 @@ int batched_tune(int kind, int prec, const Arith3& ar, const double* x, const do
     int best = 0;
     for (int v = 0; v < NVARIANT && rc == GPK_OK; ++v) {
       const Variant vr = variant_of(v);
+      const int same = variant_id(variant_for(vr, base == GPK_PREC_FP64, g.np, d));
+      if (same != v) {  // runs what an earlier one ran (variant_for only clears bits)
+        ms[v] = ms[same];
+        continue;
+      }
       rc = run_group<TS>(kind, ar, x, y, d, theta, nls, jitter, iters, ws, P, g, vr, result,
                          grad, s);
       if (rc == GPK_OK && hipEventRecord(e0, s) != hipSuccess) {

@@ -363,7 +363,10 @@ int gpk_batched_mll_grad(int kind, int prec, const double* x, const double* y,
  * leaves as the chosen variants compute them.  report_host (optional): 7 floats
  * per group, up to report_len floats -- padded size, members, chosen variant
  * (bit 0: stored Sigma, bit 1: transposed pass), then the four variants' mean
- * milliseconds.  No counterpart in the reference (XLA compiles one program per
+ * milliseconds.  In float64 some are one and the same and are timed once, their time
+ * reported for each: the transposed pass is the column-read one up to d = 32 and 4,352
+ * padded rows, and the stored Sigma the recomputed one at 128 padded rows and d <= 16.
+ * No counterpart in the reference (XLA compiles one program per
  * shape).
  */
 int gpk_batched_tune(int kind, int prec, const double* x, const double* y,

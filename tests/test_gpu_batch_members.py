@@ -46,3 +46,31 @@ def test_member_bits_do_not_depend_on_the_batch(cuda, monkeypatch, precision, n,
         rest = list(range(1, count))
         assert torch.equal(run([0] + rest)[0], alone), count
         assert torch.equal(run(rest + [0])[-1], alone), count
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_tuner_times_what_runs(cuda, precision):
+    """Variants that run the same kernels at a size are timed once and the plainer one is
+    chosen: in float64 the gradient pass reads columns whatever the variant (d <= 32),
+    and the solve of one leaf (n <= 128, d <= 16) evaluates Sigma itself, so a stored
+    copy would be written for nothing.  The mixed path has all four."""
+    rng = np.random.default_rng(3)
+    sizes = [60, 100, 129, 500, 900]
+    for d in (5, 18):
+        Xs = [rng.uniform(0.0, 1.0, (n, d)) for n in sizes]
+        ys = [np.sin(6 * X[:, 0]) for X in Xs]
+        m = gpx.batched.BatchedConjugateMLL(Xs, ys, kernel="matern12", lengthscale=1.0,
+                                            obs_stddev=0.2, precision=precision)
+        assert [r["padded_size"] for r in m.tune_report] == [128, 256, 512, 1024]
+        for r in m.tune_report:
+            ms = r["ms"]
+            assert all(t > 0 for t in ms.values())
+            if precision == "mixed":
+                assert len(set(ms.values())) > 1
+                continue
+            assert not r["transposed_pass"]
+            assert ms["recomputed/transposed"] == ms["recomputed/columns"]
+            assert ms["stored/transposed"] == ms["stored/columns"]
+            if r["padded_size"] == 128 and d <= 16:
+                assert not r["stored_sigma"]
+                assert ms["stored/columns"] == ms["recomputed/columns"]
