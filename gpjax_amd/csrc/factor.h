@@ -29,31 +29,33 @@ inline int64_t split_point(int64_t n) { return (n / NB / 2) * NB; }
 // (wide batches take the 128 x 128 tiles: 4,096 small GPs 62.3 -> 61.1 ms).
 constexpr int64_t TRSM_STRIP_TILES = 512;
 static_assert(TRSM_STRIP_TILES >= SMALL_TILES, "an in-place product on small tiles would race");
-constexpr unsigned TRI_NODEWISE = 64;  // members from which the inverse goes node by node
 
 // Largest single float64 problem factored leaf by leaf on one stream
 // (Factor::potrf_steps).  Beyond it the trailing updates, a rank-128 step each, take
 // longer than the leaf they run beside.  MLL + gradient (two streams with the
-// look-ahead / leaf by leaf with the inverse in the sweep, ms): n = 2,000 1.41 / 0.85,
-// n = 3,001 (leave-one-out) 3.16 / 2.42, n = 4,000 3.80 / 3.25; with the inverse after
-// the factor on both sides: n = 6,000 8.5 / 8.7, n = 8,000 15.6 / 17.3.
+// look-ahead and the inverse after it / leaf by leaf with the inverse in the sweep, ms):
+// n = 2,000 1.41 / 0.85, n = 3,000 2.42 / 1.75, n = 4,000 3.81 / 3.23, n = 4,500 5.14 /
+// 4.55, n = 5,000 6.12 / 5.91, n = 6,000 8.56 / 8.89, n = 8,000 15.6 / 19.6.
 constexpr int64_t STEPS_MAX = 4096;
 
 // Panel width of the look-ahead Cholesky (Factor::potrf_lookahead) for a single
 // np x np problem, np >= 2,048 (float64: > STEPS_MAX): np/32 with float32 storage, np/64
-// in float64,
-// rounded down to a multiple of NB, at least NB.  Wider panels put more of the
+// in float64, rounded down to a multiple of NB, at least NB.  Wider panels put more of the
 // update into large rank-B GEMMs; narrower ones shorten the second stream's
 // chain per panel, which the first and last panels wait for.  Measured (ms per
-// MLL + gradient, float32 storage / float64; * = the rule's choice):
-//   np =  2,048: no look-ahead 2.96 / 6.1, B = 256 2.86 / 5.5, 128 2.76* / 5.1*
-//   np =  4,096: no look-ahead 6.16 / 14.1, B = 256 5.53 / 11.7, 128 5.31* / 10.8*
-//   np =  8,192: B = 2,048 15.8 / 35.1, 512 13.9 / 30.6, 256 12.9* / 28.4,
-//                128 13.1 / 27.2*
-//   np = 16,384: B = 2,048 50.3 / 123.5, 1,024 45.9 / 117.5, 512 44.4* / 113.1,
-//                256 47.3 / 109.0*, 128 57.9 / 114.7
-//   np = 32,768: B = 2,048 227.3 / 662.5, 1,024 225.1* / 655.7, 512 239.3 / 652.5*
-//   np = 65,536: B = 4,096 1,521 / 4,602, 2,048 1,525* / 4,589, 1,024 1,576 / 4,592*
+// MLL + gradient; * = the rule's choice):
+//   float32 storage   np =  2,048: no look-ahead 1.87, B = 128 1.64*, 256 1.86
+//                     np =  4,096: no look-ahead 4.13, 128 3.24*, 256 3.75
+//                     np =  8,192: no look-ahead 11.6, 128 9.81, 256 9.35*, 512 9.99
+//                     np = 16,384: 128 53.4, 256 42.2, 512 39.0*, 1,024 39.7
+//                     np = 32,768: 512 230.8, 1,024 217.7*, 2,048 218.1
+//                     np = 65,536: 1,024 1,576, 2,048 1,525*, 4,096 1,521
+//   float64           np =  8,192: no look-ahead 17.8, 128 16.1*, 256 15.5, 512 16.3
+//                     np = 16,384: 128 95.6, 256 87.3*, 512 88.0, 1,024 88.6
+//                     np = 32,768: 512 596.9*, 1,024 592.3, 2,048 594.9
+//                     np = 65,536: 1,024 4,592*, 2,048 4,589, 4,096 4,602
+// (65,536: with the column-sweep leaf.  In float64 np/32 would now be 4 % better at 8,192
+// and no worse above.)
 // GPK_LOOKAHEAD_B set at build time fixes the width (0 turns the look-ahead off).
 #ifndef GPK_LOOKAHEAD_B
 #define GPK_LOOKAHEAD_B -1
@@ -95,7 +97,7 @@ struct Factor {
   TS* L;             // matrix in, factor out (lower NB-tiles), leading dimension ld
   TS* X;             // L^-1 out (lower)
   int64_t ld;
-  TS* T;             // scratch of (n - split(n)) * split(n) elements
+  TS* T;             // scratch of factor_scratch_elems(n) elements
   double* leafinv;   // n/NB blocks of NB x NB float64 leaf inverses
   double* leafld;    // n/NB leaf log-determinants
   int* leafinfo;     // n/NB leaf pivot status
@@ -118,12 +120,15 @@ struct Factor {
   int64_t tri_unit = NB;
 
   double* dblk_at(int64_t o) const { return dblk ? dblk + (o / NB) * NB * NB : nullptr; }
-  // Float64 with every sum in the order of its index (ar_potrf = ar_trtri = AR_F64_SEQ,
-  // no batch): the column-sweep leaf, 128-tiles, the recursion or the look-ahead.  For
-  // matrices whose inverse is then rounded to float32 (the mixed collapsed bound's G_P):
-  // a last-bit change of the order moves some of its entries to the other float32
-  // neighbour, and the gradient in Z, a difference of large terms, by 1e-9 to 6e-9.
-  // N = 1e6, M = 2,048: 79.4 ms, against 75.7 on the faster routes.
+  // Float64 with one fixed grouping of its sums (ar_potrf = ar_trtri = AR_F64_SEQ, no
+  // batch): the column-sweep leaf, 128-tiles whose products take four consecutive k, the
+  // recursion or the look-ahead.  For the mixed collapsed bound, which rounds G_P, made
+  // of these inverses, to float32: another grouping moves some of its entries to the
+  // other float32 neighbour, and the gradient in Z, a difference of large terms, by
+  // 1e-13 to 1e-7 of its norm.  That keeps results as they were, and no more: the two
+  // groupings are equally far from the float64 bound (N = 1e6, M = 2,048: 9.191e-6 of
+  // the gradient in Z both, 7.0e-9 apart), and this one takes 79.4 ms there against 75.7
+  // on the faster routes.
   bool seq() const { return ar_potrf == AR_F64_SEQ; }
   int factor_seq(int64_t n, bool streams) {
     GPK_TRY(factor_only(n, streams));
@@ -274,50 +279,32 @@ struct Factor {
   }
   // X = L^-1 below the leaves, whose diagonal blocks the leaves already wrote:
   // level by level from the deepest, all nodes of a level (independent of each
-  // other) in one launch per product, or for a wide batch, whose single nodes
-  // fill the chip, node by node (a node's T and X are then still in cache when its
-  // second product and its parent read them: 4,096 small GPs 61.7 -> 60.2 ms).
-  // n = 2,000: 30 launches of one to 64 workgroups 1,217 us, eight launches 195 us.
+  // other) in one launch per product.  The inverse of a float64 factor of 2,000 rows:
+  // 30 launches of one to 64 workgroups 1,217 us, eight launches 195 us.  (Node by node
+  // is no faster for wide batches either: 4,096 GPs of 32 to 1,024 rows 58.9 ms, 59.1
+  // by levels, and from 8 to 1,000 of 512 or 1,024 rows within 1.5 % both ways.)
   int trtri(int64_t o, int64_t n) {
-    const int depth = tri_depth((int)n, (int)tri_unit);
-    if (bt.count >= TRI_NODEWISE) return trtri_node(o, n, 0, 0);
-    for (int d = depth - 1; d >= 0; --d) GPK_TRY(trtri_level(o, n, d, 0, 1u << d));
-    return GPK_OK;
-  }
-  // Nodes first .. first + count - 1 of a level of the inverse over rows o .. o + n.
-  int trtri_level(int64_t o, int64_t n, int depth, unsigned first, unsigned count) {
     TriLevel lev;
-    lev.nodes = 1u << depth;
-    lev.depth = depth;
     lev.o = (int)o;
     lev.n = (int)n;
     lev.unit = (int)tri_unit;
     lev.ld = (int)ld;
-    int mm, mn;
-    tri_extents(lev, mm, mn);
-    lev.tstride = depth == 0 ? 0 : mn;
-    lev.first = first;
-    lev.nodes = count;
-    // T = L21 X11   ((n-h) x h; X11 lower, so k >= column tile)
-    lev.product = 1;
-    GPK_TRY(launch_tri_level<TS>(ar_trtri, lev, mm, mn, L, ld, X, ld, T, mn, s, bt,
-                                 fscale ? fscale + 1 : nullptr));
-    // X21 = -X22 T  (X22 lower, so k <= row tile)
-    lev.product = 2;
-    return launch_tri_level<TS>(ar_trtri, lev, mm, mn, X, ld, T, mn, X, ld, s, bt,
-                                fscale ? fscale + 2 : nullptr);
-  }
-  int trtri_node(int64_t o, int64_t n, unsigned path, int d) {
-    TriLevel lev;
-    lev.depth = d;
-    lev.o = (int)o;
-    lev.n = (int)n;
-    lev.unit = (int)tri_unit;
-    int no, nn, h;
-    if (!tri_node(lev, path, no, nn, h)) return GPK_OK;
-    GPK_TRY(trtri_node(o, n, 2 * path, d + 1));
-    GPK_TRY(trtri_node(o, n, 2 * path + 1, d + 1));
-    return trtri_level(o, n, d, path, 1);
+    for (int d = tri_depth((int)n, (int)tri_unit) - 1; d >= 0; --d) {
+      lev.nodes = 1u << d;
+      lev.depth = d;
+      int mm, mn;
+      tri_extents(lev, mm, mn);
+      lev.tstride = d == 0 ? 0 : mn;
+      // T = L21 X11   ((n-h) x h; X11 lower, so k >= column tile)
+      lev.product = 1;
+      GPK_TRY(launch_tri_level<TS>(ar_trtri, lev, mm, mn, L, ld, X, ld, T, mn, s, bt,
+                                   fscale ? fscale + 1 : nullptr));
+      // X21 = -X22 T  (X22 lower, so k <= row tile)
+      lev.product = 2;
+      GPK_TRY(launch_tri_level<TS>(ar_trtri, lev, mm, mn, X, ld, T, mn, X, ld, s, bt,
+                                   fscale ? fscale + 2 : nullptr));
+    }
+    return GPK_OK;
   }
 };
 

@@ -273,7 +273,8 @@ enum KRange { KR_FULL = 0, KR_GE_N = 1, KR_LE_M = 2, KR_GE_M = 3 };
 // Product arithmetic of the tile GEMM.  AR_FP16X3: float32 operands scaled by a
 // power of two (so that every entry sits well inside the fp16 range), split
 // into fp16 hi + lo planes, products hi*hi + hi*lo + lo*hi.
-// AR_F64_SEQ: float64 on 128-tiles alone, four consecutive k per product (Factor::seq).
+// AR_F64_SEQ: float64 on 128-tiles alone, four consecutive k per matrix-core product
+// (Factor::seq).
 enum Arith { AR_F64 = 0, AR_F64_SEQ = 1, AR_BF16X3 = 3, AR_FP16X3 = 4, AR_BF16X6 = 6 };
 
 // Tile rule of the FP64 products (double operands, no diagonal side buffer), by the
@@ -282,7 +283,9 @@ enum Arith { AR_F64 = 0, AR_F64_SEQ = 1, AR_BF16X3 = 3, AR_FP16X3 = 4, AR_BF16X6
 // TINY_TILES on 32 x 32.  The line lies where 128-tiles fill the chip's two
 // workgroups per CU; MLL + gradient at n = 5,000: 6.57 ms with 160, 6.45 with 384,
 // 6.19 with 512, 6.27 with 1,024 (10.9 without), n = 16,384: 86.5 / 86.8 / 86.7 /
-// 87.3 (100.9).  TINY_TILES 8, 24 and 64 are within 1 %.  In a batch the other
+// 87.3 (100.9).  The 32-wide ones (none / up to 8 / 24 / 64 tiles): n = 500 296 / 279 /
+// 278 / 279 us, n = 2,000 933 / 889 / 846 / 846, n = 4,000 3,332 / 3,290 / 3,235 / 3,221,
+// predictive at n = 2,000 with 500 points 1,247 / 1,189 / 1,107 / 1,120.  In a batch the other
 // pieces' launches fill the chip, so there only launches of few tiles take the small
 // ones (512 GPs of up to 600 rows: 3.17 ms with 512, 2.96 with 96).
 constexpr int64_t SMALL_TILES = 512, SMALL_TILES_BATCH = 96;
@@ -306,7 +309,7 @@ int launch_gemm(int arith, bool a_km, bool b_kn, const TA* A, int64_t lda, const
 // X21 = -X22 T (product 2); its T sits at T + (node's o - o) * tstride.
 struct TriLevel {
   unsigned nodes = 0;  // nodes of this launch; 0: not a level of the inverse
-  unsigned first = 0;  // the first of them
+  unsigned first = 0;  // the first of them (a level may take several launches)
   int depth = 0;
   int product = 0;
   int o = 0, n = 0, unit = NB;  // 32 bits: a kernel argument of every tile GEMM
